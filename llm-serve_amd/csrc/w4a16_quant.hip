@@ -137,25 +137,47 @@ __global__ __launch_bounds__(kQuantThreads) void quantize_kernel(const void* __r
   }
 }
 
-// Fast path for GS in {32, 64, 128} (the same arithmetic, bit for bit): each of the four
-// threads of a row holds its GS / 4 consecutive values in registers (16-byte loads), the
-// row's min and max come from two lane shuffles, and only the 4-bit codes go through LDS
-// (one byte each, rows padded to GS + 4 bytes so that the eight rows one packed word
-// gathers sit in different banks) for the transposed packing.
+// Fast path for GS in {32, 64, 128} (the same results, bit for bit): 128 output rows per
+// workgroup, four threads per row, each holding its GS / 4 consecutive values in registers
+// (16-byte loads); the row's min and max come from two lane shuffles.  Only the 4-bit codes
+// go through LDS, one byte each, for the transposed packing: a thread reads four consecutive
+// input positions of eight rows as eight words, merges them nibble by nibble and transposes
+// the four bytes by permutes into four output words (12 vector instructions for 32 codes);
+// 16 threads write the 64 consecutive bytes of an input row's words.
+//
+// Bound: the weight's read and the code's write once the arithmetic is out of the way.  An
+// IEEE division per weight (11 instructions), NaN-aware compares and the packing of single
+// bytes made about 32 vector instructions per weight, 64 us of issue for 24576 x 4096 bf16,
+// where the 254 MB take 50 us at the copy rate.  Here w / s is w times the row's reciprocal,
+// and the quotient is divided out only where that could round differently (below): about 10.
+constexpr int kFastRows = 128;
+constexpr int kFastThreads = 4 * kFastRows;
+
+// Smaller / larger of two, NaN if either is (torch's amin / amax), one instruction each.
+__device__ __forceinline__ float min_nan(float a, float b) { return __builtin_elementwise_minimum(a, b); }
+__device__ __forceinline__ float max_nan(float a, float b) { return __builtin_elementwise_maximum(a, b); }
+
+// clamp(n + z, 0, 15) as byte `e` of `word` (n, z whole numbers; the conversion clamps below
+// at 0 and takes NaN to 0).
+template <int E>
+__device__ __forceinline__ uint32_t put_code(uint32_t word, float n, float z) {
+  return __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fminf(n + z, 15.f), E, word);
+}
+
 template <int GS, int DTYPE>
-__global__ __launch_bounds__(kQuantThreads) void quantize_rows_kernel(const void* __restrict__ weight,
-                                                                      uint32_t* __restrict__ qweight,
-                                                                      uint32_t* __restrict__ qzeros,
-                                                                      void* __restrict__ scales, int out_f, int in_f) {
+__global__ __launch_bounds__(kFastThreads) void quantize_rows_kernel(const void* __restrict__ weight,
+                                                                     uint32_t* __restrict__ qweight,
+                                                                     uint32_t* __restrict__ qzeros,
+                                                                     void* __restrict__ scales, int out_f, int in_f) {
   constexpr int PART = GS / 4;       // values per thread
   constexpr int QP = GS + 4;         // LDS row pitch of the codes, bytes
   constexpr int PER = DTYPE == kDtypeF32 ? 4 : 8;  // values per 16-byte load
-  static_assert(PART % PER == 0, "a thread's values must split into 16-byte loads");
-  __shared__ __attribute__((aligned(16))) uint8_t codes[kQuantRows * QP];
-  __shared__ float row_z[kQuantRows];
-  const int o0 = blockIdx.x * kQuantRows;
+  static_assert(PART % PER == 0 && PART % 8 == 0, "a thread's values must split into 16-byte loads");
+  __shared__ __attribute__((aligned(16))) uint8_t codes[kFastRows * QP];
+  __shared__ float row_z[kFastRows];
+  const int o0 = blockIdx.x * kFastRows;
   const int g = blockIdx.y;
-  const int rows = out_f - o0 < kQuantRows ? out_f - o0 : kQuantRows;  // a multiple of 8
+  const int rows = out_f - o0 < kFastRows ? out_f - o0 : kFastRows;  // a multiple of 8
   const int tid = threadIdx.x;
   const int r = tid >> 2;  // the four threads of row r are adjacent lanes of one wave
   const int h = tid & 3;
@@ -166,86 +188,108 @@ __global__ __launch_bounds__(kQuantThreads) void quantize_rows_kernel(const void
 #pragma unroll
   for (int c = 0; c < PART; c += PER) {
     if constexpr (DTYPE == kDtypeF32) {
-      const float4 w = live ? *reinterpret_cast<const float4*>(static_cast<const float*>(weight) + base + c)
-                            : float4{0.f, 0.f, 0.f, 0.f};
+      const float4 w = *reinterpret_cast<const float4*>(static_cast<const float*>(weight) + base + c);
       v[c] = w.x; v[c + 1] = w.y; v[c + 2] = w.z; v[c + 3] = w.w;
     } else {
-      const uint4 w = live ? *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(weight) + base + c)
-                           : uint4{0u, 0u, 0u, 0u};
+      const uint4 w = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(weight) + base + c);
       const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const uint16_t lo = static_cast<uint16_t>(ww[e] & 0xFFFFu), hi = static_cast<uint16_t>(ww[e] >> 16);
         if constexpr (DTYPE == kDtypeF16) {
-          v[c + 2 * e] = static_cast<float>(__builtin_bit_cast(_Float16, lo));
-          v[c + 2 * e + 1] = static_cast<float>(__builtin_bit_cast(_Float16, hi));
+          v[c + 2 * e] = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(ww[e] & 0xFFFFu)));
+          v[c + 2 * e + 1] = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(ww[e] >> 16)));
         } else {
-          v[c + 2 * e] = bf16_bits_to_f32(lo);
-          v[c + 2 * e + 1] = bf16_bits_to_f32(hi);
+          v[c + 2 * e] = __uint_as_float(ww[e] << 16);
+          v[c + 2 * e + 1] = __uint_as_float(ww[e] & 0xFFFF0000u);
         }
       }
     }
   }
-  // Row min and max (NaN propagates as in torch's amin / amax).
   float mn = v[0], mx = v[0];
 #pragma unroll
   for (int c = 1; c < PART; ++c) {
-    mn = (v[c] < mn || v[c] != v[c]) ? v[c] : mn;
-    mx = (v[c] > mx || v[c] != v[c]) ? v[c] : mx;
+    mn = min_nan(mn, v[c]);
+    mx = max_nan(mx, v[c]);
   }
 #pragma unroll
   for (int d = 1; d <= 2; d <<= 1) {
-    const float mn2 = __shfl_xor(mn, d);
-    const float mx2 = __shfl_xor(mx, d);
-    mn = (mn2 < mn || mn2 != mn2) ? mn2 : mn;
-    mx = (mx2 > mx || mx2 != mx2) ? mx2 : mx;
+    mn = min_nan(mn, __shfl_xor(mn, d));
+    mx = max_nan(mx, __shfl_xor(mx, d));
   }
   float dd = mx - mn;
   dd = dd < 1e-5f ? 1e-5f : dd;  // torch clamp(min=): NaN stays NaN
   const float s = dd / 15.0f;
   float z = -__builtin_rintf(mn / s);
   z = z < 0.f ? 0.f : (z > 15.f ? 15.f : z);
-  if (live) {
-    uint32_t packed[PART / 4];
+
+  // Codes, eight values at a time.  t = w * (1 / s) is within 2^-23 |w / s| of w / s rounded
+  // once and again, so where the code is not clamped anyway (|w / s| < 17) the two lie within
+  // 4e-6 of each other and round to the same whole number unless t is that close to a half:
+  // then the eight are divided out.
+  const float inv = 1.0f / s;
+  uint32_t* dst = reinterpret_cast<uint32_t*>(codes + r * QP + h * PART);
 #pragma unroll
-    for (int c = 0; c < PART; c += 4) {
+  for (int c = 0; c < PART; c += 8) {
+    float n[8];
+    float off = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float t = v[c + e] * inv;
+      n[e] = __builtin_rintf(t);
+      off = __builtin_fmaxf(off, __builtin_fabsf(t - n[e]));
+    }
+    if (off > 0.49999f) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) n[e] = __builtin_rintf(v[c + e] / s);
+    }
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
       uint32_t word = 0;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float q = __builtin_rintf(v[c + e] / s) + z;
-        q = q < 0.f ? 0.f : (q > 15.f ? 15.f : q);
-        word |= (static_cast<uint32_t>(q) & 0xFFu) << (8 * e);
-      }
-      packed[c / 4] = word;
+      word = put_code<0>(word, n[4 * q], z);
+      word = put_code<1>(word, n[4 * q + 1], z);
+      word = put_code<2>(word, n[4 * q + 2], z);
+      word = put_code<3>(word, n[4 * q + 3], z);
+      dst[c / 4 + q] = word;
     }
-    uint32_t* dst = reinterpret_cast<uint32_t*>(codes + r * QP + h * PART);
-#pragma unroll
-    for (int c = 0; c < PART / 4; ++c) dst[c] = packed[c];
-    if (h == 0) {
-      row_z[r] = z;
-      const size_t si = static_cast<size_t>(g) * out_f + o0 + r;
-      if constexpr (DTYPE == kDtypeF32) static_cast<float*>(scales)[si] = s;
-      else if constexpr (DTYPE == kDtypeF16) static_cast<_Float16*>(scales)[si] = static_cast<_Float16>(s);
-      else static_cast<uint16_t*>(scales)[si] = f32_to_bf16_bits(s);
-    }
+  }
+  if (live && h == 0) {
+    row_z[r] = z;
+    const size_t si = static_cast<size_t>(g) * out_f + o0 + r;
+    if constexpr (DTYPE == kDtypeF32) static_cast<float*>(scales)[si] = s;
+    else if constexpr (DTYPE == kDtypeF16) static_cast<_Float16*>(scales)[si] = static_cast<_Float16>(s);
+    else static_cast<uint16_t*>(scales)[si] = f32_to_bf16_bits(s);
   }
   __syncthreads();
 
-  const int W = rows / 8;    // packed words per input row in this workgroup
-  const int C8 = out_f / 8;  // packed words per input row
-  if (tid < W) {
+  constexpr int W = kFastRows / 8;  // packed words per input row in this workgroup
+  const int words = rows / 8;       // those inside the weight
+  const int C8 = out_f / 8;         // packed words per input row
+  if (tid < words) {
     uint32_t word = 0;
 #pragma unroll
     for (int c = 0; c < 8; ++c) word |= (static_cast<uint32_t>(row_z[8 * tid + c]) & 0xFu) << awq_shift(c);
     qzeros[static_cast<size_t>(g) * C8 + o0 / 8 + tid] = word;
   }
-  for (int e = tid; e < GS * W; e += kQuantThreads) {
-    const int k = e / W;
-    const int j = e - k * W;
-    uint32_t word = 0;
 #pragma unroll
-    for (int c = 0; c < 8; ++c) word |= (static_cast<uint32_t>(codes[(8 * j + c) * QP + k]) & 0xFu) << awq_shift(c);
-    qweight[(static_cast<size_t>(g) * GS + k) * C8 + o0 / 8 + j] = word;
+  for (int e = tid; e < GS / 4 * W; e += kFastThreads) {
+    const int k4 = e / W;
+    const int j = e % W;
+    if (j >= words) continue;
+    // Row c's codes of positions 4 k4 .. + 3; columns 0, 2, 4, 6 of an AutoAWQ word are the
+    // nibbles of its low half, 1, 3, 5, 7 those of its high half.
+    uint32_t row[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) row[c] = *reinterpret_cast<const uint32_t*>(codes + (8 * j + c) * QP + 4 * k4);
+    const uint32_t b0 = row[0] | (row[2] << 4), b1 = row[4] | (row[6] << 4);
+    const uint32_t b2 = row[1] | (row[3] << 4), b3 = row[5] | (row[7] << 4);
+    // byte i of (b0, b1, b2, b3) -> word i (v_perm_b32 selects among the 8 bytes of hi:lo)
+    const uint32_t lo01 = __builtin_amdgcn_perm(b1, b0, 0x05010400u), hi01 = __builtin_amdgcn_perm(b1, b0, 0x07030602u);
+    const uint32_t lo23 = __builtin_amdgcn_perm(b3, b2, 0x05010400u), hi23 = __builtin_amdgcn_perm(b3, b2, 0x07030602u);
+    uint32_t* out = qweight + (static_cast<size_t>(g) * GS + 4 * k4) * C8 + o0 / 8 + j;
+    out[0] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
+    out[C8] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
+    out[2 * static_cast<size_t>(C8)] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
+    out[3 * static_cast<size_t>(C8)] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
   }
 }
 
@@ -269,16 +313,17 @@ size_t quantize_lds_bytes(int group_size) {
 
 template <int GS>
 static hipError_t launch_quantize_rows(const void* weight, int dtype, uint32_t* qweight, uint32_t* qzeros,
-                                       void* scales, int out_f, int in_f, dim3 grid, hipStream_t stream) {
+                                       void* scales, int out_f, int in_f, hipStream_t stream) {
+  const dim3 grid((out_f + kFastRows - 1) / kFastRows, in_f / GS);
   switch (dtype) {
     case kDtypeF32:
-      quantize_rows_kernel<GS, kDtypeF32><<<grid, kQuantThreads, 0, stream>>>(weight, qweight, qzeros, scales, out_f, in_f);
+      quantize_rows_kernel<GS, kDtypeF32><<<grid, kFastThreads, 0, stream>>>(weight, qweight, qzeros, scales, out_f, in_f);
       break;
     case kDtypeF16:
-      quantize_rows_kernel<GS, kDtypeF16><<<grid, kQuantThreads, 0, stream>>>(weight, qweight, qzeros, scales, out_f, in_f);
+      quantize_rows_kernel<GS, kDtypeF16><<<grid, kFastThreads, 0, stream>>>(weight, qweight, qzeros, scales, out_f, in_f);
       break;
     default:
-      quantize_rows_kernel<GS, kDtypeBF16><<<grid, kQuantThreads, 0, stream>>>(weight, qweight, qzeros, scales, out_f, in_f);
+      quantize_rows_kernel<GS, kDtypeBF16><<<grid, kFastThreads, 0, stream>>>(weight, qweight, qzeros, scales, out_f, in_f);
   }
   return hipGetLastError();
 }
@@ -289,9 +334,9 @@ hipError_t launch_quantize(const void* weight, int dtype, uint32_t* qweight, uin
   // Fast path: 16-byte aligned weight (every row segment a thread loads is then aligned).
   if (reinterpret_cast<uintptr_t>(weight) % 16 == 0) {
     switch (group_size) {
-      case 128: return launch_quantize_rows<128>(weight, dtype, qweight, qzeros, scales, out_f, in_f, grid, stream);
-      case 64: return launch_quantize_rows<64>(weight, dtype, qweight, qzeros, scales, out_f, in_f, grid, stream);
-      case 32: return launch_quantize_rows<32>(weight, dtype, qweight, qzeros, scales, out_f, in_f, grid, stream);
+      case 128: return launch_quantize_rows<128>(weight, dtype, qweight, qzeros, scales, out_f, in_f, stream);
+      case 64: return launch_quantize_rows<64>(weight, dtype, qweight, qzeros, scales, out_f, in_f, stream);
+      case 32: return launch_quantize_rows<32>(weight, dtype, qweight, qzeros, scales, out_f, in_f, stream);
       default: break;
     }
   }

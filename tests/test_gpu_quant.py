@@ -150,3 +150,28 @@ def test_adversarial_groups_bit_exact(cal, dtype, kind):
     np.testing.assert_array_equal(p.qweight.cpu().numpy(), qw)
     np.testing.assert_array_equal(p.qzeros.cpu().numpy(), qz)
     np.testing.assert_array_equal(scale_array(p.scales), sc)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("gs", [32, 64, 128])
+def test_quotients_near_half_and_row_block_edges(cal, dtype, gs):
+    """Weights whose quotient by the scale is a half exactly, or the values of the dtype next to
+    it, in groups that span [-7.5 s, 7.5 s] (ties at both ends) and [0, 15 s] for scales that
+    are powers of two, thirds and tenths: the codes come from a reciprocal except next to a half,
+    and must be the rounded quotient's everywhere.  Row counts around the 128 rows of a
+    workgroup."""
+    for rows in (8, 120, 128, 136):
+        w = torch.empty(rows, 2 * gs, dtype=torch.float64)
+        steps = torch.arange(2 * gs, dtype=torch.float64) % 31
+        for r in range(rows):
+            w[r] = [2.0 ** -6, 2.0 ** -5 / 3, 0.01, 3e-5 * (r + 1)][r % 4] * ((-7.5 if r % 8 < 4 else 0.0) + steps / 2)
+        w = w.to(dtype)
+        bits = w.view(torch.int16 if w.element_size() == 2 else torch.int32)
+        bits[:, 3::4] += (bits[:, 3::4] != 0).to(bits.dtype)  # the next value away from zero
+        bits[:, 2::4] -= (bits[:, 2::4] != 0).to(bits.dtype)  # and towards it
+        print(f"quantize near halves {dtype} rows={rows} g{gs}", flush=True)
+        p = cal.quantize_awq_weight(w.cuda(), group_size=gs)
+        qw, qz, sc = ora.quantize_awq_weight(w.float().numpy(), group_size=gs, out_dtype=ORACLE_DTYPE[dtype])
+        np.testing.assert_array_equal(p.qweight.cpu().numpy(), qw)
+        np.testing.assert_array_equal(p.qzeros.cpu().numpy(), qz)
+        np.testing.assert_array_equal(scale_array(p.scales), sc)
