@@ -57,33 +57,78 @@ __global__ __launch_bounds__(256) void dequant_awq_kernel(const uint32_t* __rest
   *reinterpret_cast<uint4*>(w_out + idx * 8) = make_uint4(outw[0], outw[1], outw[2], outw[3]);
 }
 
-// One thread per output word of the group-tile layout (see w4a16_common.h): gathers the
-// 8 nibbles it holds from two AutoAWQ words (rows r and r + 4, the same 4 columns).
-// Writes are coalesced; this runs once per weight at load time.
+// AutoAWQ words -> the group-tile layout (see w4a16_common.h), one workgroup per (128-row
+// group, up to 16 column tiles).  The block's 128 rows x 32 words (128 consecutive bytes per
+// row) go through LDS; each thread then gathers the 16 bytes of one lane slot of a tile -- the
+// nibbles of eight words, two rows r and r + 4 for each of its four 32-row steps -- and the
+// block's tiles are one contiguous run of the output.  HBM-bound, K N bytes in all.  (A thread
+// per output word, gathering its two words from memory, read them in 8-byte pieces of rows
+// N / 2 bytes apart, four times over: 58 us for 4096 x 24576.)
+//
+// VEC: qweight and packed 16-byte aligned and rows a multiple of 16 bytes; otherwise one word
+// per load and store.
+constexpr int kRepackTiles = 16;
+constexpr int kRepackWords = 2 * kRepackTiles;   // AutoAWQ words per row of the block
+constexpr int kRepackPitch = kRepackWords + 4;   // LDS row pitch: 16-byte rows, 2-way conflicts at most
+template <bool VEC>
 __global__ __launch_bounds__(256) void repack_kernel(const uint32_t* __restrict__ qweight,
-                                                     uint32_t* __restrict__ packed, int K, int N) {
-  const size_t idx = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const size_t total = static_cast<size_t>(K) * (N >> 3);
-  if (idx >= total) return;
+                                                     uint32_t* __restrict__ packed, int N, int blocks_n) {
+  __shared__ __attribute__((aligned(16))) uint32_t rows[kGroup * kRepackPitch];
   const int NT = N / kTileCols;
-  const int js = static_cast<int>(idx & 3);
-  const int lane = static_cast<int>((idx >> 2) & 63);
-  const size_t tile = idx >> 8;
-  const int g = static_cast<int>(tile / NT);
-  const int t = static_cast<int>(tile - static_cast<size_t>(g) * NT);
-  const int col0 = kTileCols * t + 4 * ((lane >> 2) & 3);  // 4 columns of one AutoAWQ word
-  uint32_t out = 0;
+  const int C8 = N >> 3;
+  const int g = blockIdx.x / blocks_n;
+  const int t0 = (blockIdx.x - g * blocks_n) * kRepackTiles;
+  const int tiles = NT - t0 < kRepackTiles ? NT - t0 : kRepackTiles;
+  const int words = 2 * tiles;
+  const int tid = threadIdx.x;
+  const uint32_t* src = qweight + static_cast<size_t>(g) * kGroup * C8 + 2 * t0;
+  if constexpr (VEC) {  // words is a multiple of 4
+    constexpr int kPerRow = kRepackWords / 4;
+    const int c = 4 * (tid % kPerRow);
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int row = kGroup * g + 32 * js + 8 * (lane >> 4) + 4 * h + (lane & 3);
-    const uint32_t src = qweight[static_cast<size_t>(row) * (N >> 3) + (col0 >> 3)];
+    for (int i = 0; i < kGroup * kPerRow / 256; ++i) {
+      const int r = i * (256 / kPerRow) + tid / kPerRow;
+      if (c < words)
+        *reinterpret_cast<uint4*>(rows + r * kRepackPitch + c) =
+            *reinterpret_cast<const uint4*>(src + static_cast<size_t>(r) * C8 + c);
+    }
+  } else {
+    const int c = tid % kRepackWords;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const uint32_t q = (src >> awq_shift((col0 + k) & 7)) & 0xFu;
-      out |= q << (8 * h + 4 * (k >> 1) + 16 * (k & 1));
+    for (int i = 0; i < kGroup * kRepackWords / 256; ++i) {
+      const int r = i * (256 / kRepackWords) + tid / kRepackWords;
+      if (c < words) rows[r * kRepackPitch + c] = src[static_cast<size_t>(r) * C8 + c];
     }
   }
-  packed[idx] = out;
+  __syncthreads();
+  uint32_t* dst = packed + (static_cast<size_t>(g) * NT + t0) * kTileWords;
+#pragma unroll
+  for (int i = 0; i < kRepackTiles * 64 / 256; ++i) {
+    const int slot = i * 256 + tid;  // tile * 64 + lane
+    const int lane = slot & 63;
+    if (slot >= tiles * 64) break;
+    // the four columns of the lane: half of one AutoAWQ word, its columns 4 hw .. 4 hw + 3
+    const int col = 2 * (slot >> 6) + ((lane >> 3) & 1);
+    const int hw = (lane >> 2) & 1;
+    uint32_t out[4];
+#pragma unroll
+    for (int js = 0; js < 4; ++js) {
+      uint32_t w = 0;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int row = 32 * js + 8 * (lane >> 4) + 4 * h + (lane & 3);
+        // columns 4 hw + k sit at bits 8 hw + 4 (k / 2) + 16 (k % 2): the layout's own order
+        w |= ((rows[row * kRepackPitch + col] >> (8 * hw)) & 0x00FF00FFu) << (8 * h);
+      }
+      out[js] = w;
+    }
+    if constexpr (VEC) {
+      *reinterpret_cast<uint4*>(dst + 4 * slot) = make_uint4(out[0], out[1], out[2], out[3]);
+    } else {
+#pragma unroll
+      for (int js = 0; js < 4; ++js) dst[4 * slot + js] = out[js];
+    }
+  }
 }
 
 // One wave per (group, 16-column tile): the MFMA GEMMs' dequant (dequant_step) run on the
@@ -134,8 +179,12 @@ hipError_t launch_dequant(const uint32_t* qweight, const uint32_t* qzeros, const
 }
 
 hipError_t launch_repack(const uint32_t* qweight, uint32_t* packed, int K, int N, hipStream_t stream) {
-  const size_t n = static_cast<size_t>(K) * (N >> 3);
-  repack_kernel<<<blocks_for(n, 256), 256, 0, stream>>>(qweight, packed, K, N);
+  const int blocks_n = (N / kTileCols + kRepackTiles - 1) / kRepackTiles;
+  const unsigned grid = static_cast<unsigned>(K / kGroup) * static_cast<unsigned>(blocks_n);
+  const bool vec = N % 32 == 0 && reinterpret_cast<uintptr_t>(qweight) % 16 == 0 &&
+                   reinterpret_cast<uintptr_t>(packed) % 16 == 0;
+  if (vec) repack_kernel<true><<<grid, 256, 0, stream>>>(qweight, packed, N, blocks_n);
+  else repack_kernel<false><<<grid, 256, 0, stream>>>(qweight, packed, N, blocks_n);
   return hipGetLastError();
 }
 

@@ -133,3 +133,18 @@ def test_tile_dequant_bit_exact_full_shape(gpu_lib, shape):
     w_ref = awq.dequantize_awq_gemm(qw, qz, s, group_size=128)
     w_tile = gpu_lib.dequant_packed(awq.repack_awq_qweight(qw), qz, s, k, n)
     assert torch.equal(w_ref.view(torch.int16), w_tile.view(torch.int16))
+
+
+@pytest.mark.parametrize("k,n", [(128, 16), (128, 48), (256, 240), (128, 256), (256, 272), (128, 560)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_repack_block_edges(gpu_lib, k, n, offset):
+    """Blocks of up to 16 column tiles: one tile, a last block of one tile and of fifteen, whole
+    blocks; rows a multiple of 16 bytes (N % 32 == 0) or not, and a weight that starts 4 bytes
+    past a 16-byte boundary (both take single-word loads and stores)."""
+    rng = np.random.default_rng(k + n)
+    qw = rng.integers(-2 ** 31, 2 ** 31, size=(k, n // 8), dtype=np.int64).astype(np.int32)
+    store = torch.empty(k * n // 8 + 4, dtype=torch.int32, device="cuda")
+    view = store[offset:offset + k * n // 8].view(k, n // 8)
+    view.copy_(torch.from_numpy(qw))
+    assert (view.data_ptr() % 16 != 0) == bool(offset)
+    np.testing.assert_array_equal(gpu_lib.repack_qweight(view).cpu().numpy(), group_tile_layout_numpy(qw))
