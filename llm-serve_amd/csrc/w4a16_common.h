@@ -110,10 +110,17 @@ __device__ __forceinline__ float wave_sum64(float v) {
   return (r0 + r2) + (r1 + r3);
 }
 
-// 1 / sqrt(v) for the RMSNorm row scale, evaluated in fp64 and rounded once to fp32 (within
-// half an fp32 ulp but for fp64's own rounding); once per row, so fp64 costs nothing.
+// 1 / sqrt(v) for the RMSNorm row scale: the fp64 reciprocal square root instruction (within
+// 2^-24 or so) and one Newton step in fp64 -- r + r (1 - v r^2) / 2, whose error is 3/2 of the
+// first one's square, 2^-46 -- rounded once to fp32: within half an fp32 ulp but for about one
+// result in 2^20.  Four dependent fp64 operations; the correctly rounded fp64 square root and
+// quotient this replaces are some forty, at the point of the norm that every wave waits for.
+// v = 0 and v = inf, where the step is NaN, keep the instruction's inf and 0.
 __device__ __forceinline__ float rsqrt_rn(float v) {
-  return static_cast<float>(1.0 / __builtin_sqrt(static_cast<double>(v)));
+  const double d = static_cast<double>(v);
+  const double r = __builtin_amdgcn_rsq(d);
+  const double e = __builtin_fma(-d * r, r, 1.0);
+  return static_cast<float>(e == e ? __builtin_fma(0.5 * r, e, r) : r);
 }
 
 // RMSNorm scaling of one chunk of s (fp32, the residual sum): bf16(float(bf16(s * rstd)) *

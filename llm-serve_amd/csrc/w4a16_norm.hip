@@ -5,7 +5,7 @@
 // Per row of K elements, in the reference's order (layernorm.py:17-40):
 //   s  = float(x) + float(residual)            (fp32; s = float(x) without a residual)
 //   residual_out = bf16(s)
-//   r  = rsqrt(mean(s * s) + eps)               (fp32 sum of squares; rsqrt in fp64)
+//   r  = rsqrt(mean(s * s) + eps)               (fp32 sum of squares; rsqrt through fp64)
 //   x_norm = bf16(float(bf16(s * r)) * float(weight))
 // s stays in registers between the two passes (K <= kNormMaxK), so residual_out may be
 // residual or x, and x_norm may be x: every element is read by the thread that writes it,
@@ -31,14 +31,16 @@ constexpr int kNormThreads = 256;
 template <bool RES, int LPR>
 __global__ __launch_bounds__(kNormThreads) void add_rmsnorm_rows_kernel(
     const uint16_t* x, const uint16_t* residual, const uint16_t* __restrict__ weight, uint16_t* x_norm,
-    uint16_t* residual_out, int M, int K, int rows_inner, int64_t stride_outer, int64_t stride_inner, float eps) {
+    uint16_t* residual_out, int M, int K, int rows_inner, int inner_shift, int64_t stride_outer,
+    int64_t stride_inner, float eps) {
   constexpr int kRows = kNormThreads / LPR;  // rows per workgroup
   const int c = threadIdx.x % LPR;           // the lane's chunk of its row
   const int r = blockIdx.x * kRows + static_cast<int>(threadIdx.x / LPR);
   const bool on = r < M && c < (K >> 3);
-  const int64_t xrow = on ? static_cast<int64_t>(r / rows_inner) * stride_outer +
-                                static_cast<int64_t>(r % rows_inner) * stride_inner
-                          : 0;
+  // (uniform: a division only where rows_inner is no power of two, inner_shift < 0)
+  const int outer = inner_shift >= 0 ? r >> inner_shift : r / rows_inner;
+  const int64_t xrow =
+      on ? static_cast<int64_t>(outer) * stride_outer + static_cast<int64_t>(r - outer * rows_inner) * stride_inner : 0;
   const size_t row = static_cast<size_t>(on ? r : 0) * K;
   // The weight chunk is loaded first, so that it arrives during the sum of squares.
   uint4 wv{};
@@ -69,15 +71,16 @@ __global__ __launch_bounds__(kNormThreads) void add_rmsnorm_rows_kernel(
 // so a row costs one memory round trip; the stores follow the reduction (stores past the
 // row are dropped).  The row comes from blockIdx alone, so the buffer descriptors are
 // uniform over the workgroup.
-template <bool RES, int C>
+template <bool RES, int C, bool STRIDED>
 __global__ __launch_bounds__(kNormThreads) void add_rmsnorm_kernel(
     const uint16_t* x, const uint16_t* residual, const uint16_t* __restrict__ weight, uint16_t* x_norm,
     uint16_t* residual_out, int K, int rows_inner, int64_t stride_outer, int64_t stride_inner, float eps) {
   const int l = threadIdx.x;
   const int r = blockIdx.x;  // the grid has one workgroup per row
-  const int64_t xrow = static_cast<int64_t>(r / rows_inner) * stride_outer +
-                       static_cast<int64_t>(r % rows_inner) * stride_inner;
   const size_t row = static_cast<size_t>(r) * K;
+  const int64_t xrow = STRIDED ? static_cast<int64_t>(r / rows_inner) * stride_outer +
+                                     static_cast<int64_t>(r % rows_inner) * stride_inner
+                               : static_cast<int64_t>(row);
   const uint32_t row_bytes = static_cast<uint32_t>(K) * 2u;
   const auto xb = make_buffer(x + xrow, row_bytes);
   const auto rb = make_buffer(RES ? residual + row : x, RES ? row_bytes : 0u);
@@ -127,8 +130,10 @@ hipError_t launch_lpr(const uint16_t* x, const uint16_t* residual, const uint16_
                       uint16_t* residual_out, int M, int K, int rows_inner, int64_t stride_outer,
                       int64_t stride_inner, float eps, hipStream_t stream) {
   constexpr int kRows = kNormThreads / LPR;
+  const int inner_shift = rows_inner >= M ? 31  // one inner run: outer is always 0
+                          : (rows_inner & (rows_inner - 1)) == 0 ? __builtin_ctz(rows_inner) : -1;
   add_rmsnorm_rows_kernel<RES, LPR><<<(M + kRows - 1) / kRows, kNormThreads, 0, stream>>>(
-      x, residual, weight, x_norm, residual_out, M, K, rows_inner, stride_outer, stride_inner, eps);
+      x, residual, weight, x_norm, residual_out, M, K, rows_inner, inner_shift, stride_outer, stride_inner, eps);
   return hipGetLastError();
 }
 
@@ -136,8 +141,12 @@ template <bool RES, int C>
 hipError_t launch_whole(const uint16_t* x, const uint16_t* residual, const uint16_t* weight, uint16_t* x_norm,
                         uint16_t* residual_out, int M, int K, int rows_inner, int64_t stride_outer,
                         int64_t stride_inner, float eps, hipStream_t stream) {
-  add_rmsnorm_kernel<RES, C><<<M, kNormThreads, 0, stream>>>(x, residual, weight, x_norm, residual_out, K,
-                                                            rows_inner, stride_outer, stride_inner, eps);
+  if (rows_inner >= M && stride_inner == K)  // contiguous rows: no division ahead of the loads
+    add_rmsnorm_kernel<RES, C, false><<<M, kNormThreads, 0, stream>>>(x, residual, weight, x_norm, residual_out, K,
+                                                                     rows_inner, stride_outer, stride_inner, eps);
+  else
+    add_rmsnorm_kernel<RES, C, true><<<M, kNormThreads, 0, stream>>>(x, residual, weight, x_norm, residual_out, K,
+                                                                    rows_inner, stride_outer, stride_inner, eps);
   return hipGetLastError();
 }
 
