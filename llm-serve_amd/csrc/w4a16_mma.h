@@ -41,21 +41,103 @@ __device__ __forceinline__ TileCoord tile_coord(int b, int m_blocks, int n_block
   return TileCoord{sidx, grp * kGroupM + in_grp % gm, in_grp / gm};
 }
 
-// The scale pair word and the AutoAWQ zero word holding the lane's column, per tile of a
-// wave, for one group.
-template <int TW>
+// A wave's output tile of TW 16-column layout tiles x 16 WM rows, on one of two matrix
+// instructions:
+//   WIDE   v_mfma_f32_32x32x16_bf16 over blocks of 32 rows x 32 columns (pairs of layout tiles);
+//   else   v_mfma_f32_16x16x32_bf16 over blocks of 16 x 16.
+// A 32x32x16 does the work of two 16x16x32 in the same 32 cycles and takes the issue port
+// once.  Register-only loops with two waves on a SIMD and three VALU instructions per 16
+// matrix cycles -- the dequant's density where a weight serves 32 to 96 rows -- run at 18.5
+// cycles per 16 with it and at 22.3 with 16x16x32.  But it passes twice the accumulator data
+// per operation and draws more power: on random operands the chip sustains 1.84 PFLOP/s of
+// 32x32x16 and 2.10 of 16x16x32 (2.43 of either on zeros).  So the wide form serves the short
+// tiles of mid-sized batches, which wait for the issue port, and the narrow form the large
+// tiles, which run at the power limit.
+//
+// Which weights a lane of the wide form holds.  A 32x32x16 B fragment has column l % 32 in
+// lane l and K rows 8 (l / 32) .. + 7 of its 16.  Lane row r = l / 16 of a group-tile load
+// holds rows 8 r .. + 7 (of each 32) of 16 columns, and the contraction may take the K rows
+// in any order that A follows: fragment 2 js + ab of 32-row step js takes rows {8 ab ..} and
+// {16 + 8 ab ..}, so lane l loads tile pair member (l / 16) % 2, lane slot (l % 16) +
+// 32 (l / 32) + 16 ab -- a permutation of the load addresses, no data movement -- and A reads
+// the same rows' chunks 4 js + 2 (l / 32) + ab.
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef __attribute__((address_space(3))) uint8_t lds_u8_t;
+typedef __attribute__((address_space(3))) void lds_void_t;
+
+template <int WM, int TW, bool WIDE>
+struct WaveTile {
+  static constexpr bool kWide = WIDE;
+  static_assert(!WIDE || TW % 2 == 0, "pairs of layout tiles");
+  static constexpr int kTiles = TW;
+  static constexpr int kSteps = kWide ? 8 : 4;      // matrix steps of a 128-deep group
+  static constexpr int MT = kWide ? WM / 2 : WM;    // row blocks
+  static constexpr int NT = kWide ? TW / 2 : TW;    // column blocks
+  static constexpr int Q = kWide ? 4 : 1;           // 16-byte fragments per block
+  static constexpr int kRows = kWide ? 32 : 16;     // rows of a block
+  static constexpr int kCols = kWide ? 32 : 16;     // columns of a block
+  static constexpr int kFrags = MT * NT * Q;        // WM TW 16-byte fragments per lane
+  static_assert(!kWide || WM % 2 == 0, "32-row blocks");
+  typedef std::conditional_t<kWide, f32x16_t, f32x4_t> acc_t;
+  acc_t acc[MT][NT];
+
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int i = 0; i < 4 * Q; ++i) acc[mt][nt][i] = 0.f;
+  }
+  // Fragment f = (mt NT + nt) Q + q: rows row(mt, q, i), i < 4, of column col(nt).
+  __device__ __forceinline__ f32x4_t get(int f) const {
+    const acc_t& v = acc[f / (NT * Q)][f / Q % NT];
+    const int q = 4 * (f % Q);
+    return f32x4_t{v[q], v[q + 1], v[q + 2], v[q + 3]};
+  }
+  __device__ __forceinline__ void set(int f, f32x4_t x) {
+    acc_t& v = acc[f / (NT * Q)][f / Q % NT];
+    const int q = 4 * (f % Q);
+    v[q] = x[0];
+    v[q + 1] = x[1];
+    v[q + 2] = x[2];
+    v[q + 3] = x[3];
+  }
+  static __device__ __forceinline__ int row(int mt, int q, int i, int lane) {
+    return kWide ? 32 * mt + 8 * q + 4 * (lane >> 5) + i : 16 * mt + 4 * (lane >> 4) + i;
+  }
+  static __device__ __forceinline__ int col(int nt, int lane) {
+    return kWide ? 32 * nt + (lane & 31) : 16 * nt + (lane & 15);
+  }
+  // Layout tile, within the wave's TW, of the lane's column in column block nt.
+  static __device__ __forceinline__ int tile_of(int nt, int lane) { return kWide ? 2 * nt + ((lane >> 4) & 1) : nt; }
+  static __device__ __forceinline__ acc_t mfma(bf16x8_t a, bf16x8_t b, acc_t c) {
+    if constexpr (kWide) return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+    else return mfma16(a, b, c);
+  }
+};
+
+// The scale pair word and the AutoAWQ zero word holding the lane's column, per column block of
+// a wave, for one group.
+template <int NT>
 struct GroupScales {
-  uint32_t s[TW], zw[TW];
+  uint32_t s[NT], zw[NT];
 };
 
 // Raw loads of one group for a wave's TW layout tiles: one 16-byte weight load per tile,
-// and (LOAD_SC) the scale-pair and zero words of the lane's column in each tile -- else those
-// come from the workgroup's LDS stage (issue_sz_stage, read_group_scales).  Decoding waits
-// until the group is consumed.  A wave whose columns lie past N fetches nothing.
-template <int TW>
+// and (LOAD_SC) the scale-pair and zero words of the lane's columns -- else those come from
+// the workgroup's LDS stage (issue_sz_stage, read_group_scales).  Decoding waits until the
+// group is consumed.  A wave whose columns lie past N fetches nothing.
+template <class Wt>
 struct BGroup {
-  u32x4_t w[TW];
-  GroupScales<TW> sc;
+  u32x4_t w[Wt::kTiles];
+  GroupScales<Wt::NT> sc;
+  // Word of matrix step s in column block nt: the 4 words of a load are 32-row steps, and a
+  // wide block has two loads, one per half of the rows.
+  __device__ __forceinline__ uint32_t word(int nt, int s) const {
+    if constexpr (Wt::kWide) return w[2 * nt + s % 2][s / 2];
+    else return w[nt][s];
+  }
 };
 
 struct BSources {
@@ -69,23 +151,30 @@ struct BSources {
 // instruction's scalar offset and the lane's part is the same for every group, so the loop
 // spends no vector instructions on addresses; every lane offset plus its group offset stays
 // inside its buffer (the wave's tiles lie below N / 16).
-template <int TW, bool LOAD_SC>
-__device__ __forceinline__ void load_b_group(BGroup<TW>& b, const BSources& src, int g, bool active, int N, int t0,
+template <class Wt, bool LOAD_SC>
+__device__ __forceinline__ void load_b_group(BGroup<Wt>& b, const BSources& src, int g, bool active, int N, int t0,
                                              int dt, int lane) {
-  const int NT = N / kTileCols;
+  constexpr int TW = Wt::kTiles;
+  const int NT16 = N / kTileCols;
   const int c = lane & 15;
   const uint32_t oob = active ? 0u : kOutOfRange;
 #pragma unroll
-  for (int tt = 0; tt < TW; ++tt) {
+  for (int nt = 0; nt < Wt::NT; ++nt) {
+    const int tt = Wt::tile_of(nt, lane);
     const int t = t0 + tt + (tt >= TW / 2 ? dt : 0);
-    const uint32_t wo = oob | (static_cast<uint32_t>(t * 64 + lane) * 16u);
-    b.w[tt] = __builtin_amdgcn_raw_buffer_load_b128(src.w, wo, static_cast<int>(static_cast<uint32_t>(g) * NT * 1024u),
-                                                     0);
+    const int gw = static_cast<int>(static_cast<uint32_t>(g) * NT16 * 1024u);
+    if constexpr (Wt::kWide) {
+      const uint32_t wo = oob + static_cast<uint32_t>(t * 64 + (lane & 47)) * 16u;
+      b.w[2 * nt] = __builtin_amdgcn_raw_buffer_load_b128(src.w, wo, gw, 0);
+      b.w[2 * nt + 1] = __builtin_amdgcn_raw_buffer_load_b128(src.w, wo + 256u, gw, 0);
+    } else {
+      b.w[nt] = __builtin_amdgcn_raw_buffer_load_b128(src.w, oob | (static_cast<uint32_t>(t * 64 + lane) * 16u), gw, 0);
+    }
     if constexpr (LOAD_SC) {
       const int col = kTileCols * t + c;
-      b.sc.s[tt] = __builtin_amdgcn_raw_buffer_load_b32(src.s, oob | (static_cast<uint32_t>(col & ~1) * 2u),
+      b.sc.s[nt] = __builtin_amdgcn_raw_buffer_load_b32(src.s, oob | (static_cast<uint32_t>(col & ~1) * 2u),
                                                         static_cast<int>(static_cast<uint32_t>(g) * N * 2u), 0);
-      b.sc.zw[tt] = __builtin_amdgcn_raw_buffer_load_b32(src.z, oob | (static_cast<uint32_t>(col >> 3) * 4u),
+      b.sc.zw[nt] = __builtin_amdgcn_raw_buffer_load_b32(src.z, oob | (static_cast<uint32_t>(col >> 3) * 4u),
                                                          static_cast<int>(static_cast<uint32_t>(g) * (N >> 3) * 4u), 0);
     }
   }
@@ -109,9 +198,8 @@ constexpr int sz_zero_chunks() { return (BN + 63) / 64; }
 // last group): its part of the offset is the instruction's scalar offset, the lane's part
 // (the column) the same for every group.
 template <int BN>
-__device__ __forceinline__ void issue_sz_stage(const BSources& src, uint8_t* sz, int g, int N, int cs0, int cs1,
+__device__ __forceinline__ void issue_sz_stage(const BSources& src, lds_u8_t* sz, int g, int N, int cs0, int cs1,
                                                int which, int lane) {
-  typedef __attribute__((address_space(3))) void lds_void_t;
   static_assert(BN % 32 == 0 && BN / 8 <= 64, "one instruction holds the scales of the column block");
   if (which == 0) {
     constexpr int kHalf = BN / 16;  // 16-byte chunks of one range
@@ -136,13 +224,15 @@ __device__ __forceinline__ void issue_sz_stage(const BSources& src, uint8_t* sz,
 // [16 TW wn, 16 TW (wn + 1)) of the block; fused, even TW: gate columns [8 TW wn, 8 TW (wn + 1))
 // of range 0 and the same up columns of range 1; fused, odd TW: columns [16 TW v, 16 TW (v + 1))
 // of range 0 for the first half of the waves (v = wn) and of range 1 for the second.
-template <int TW, int BN>
+template <class Wt, int BN>
 struct SzOffsets {
-  uint32_t s[TW], z[TW];
+  static constexpr int TW = Wt::kTiles, NT = Wt::NT;
+  uint32_t s[NT], z[NT];
   __device__ __forceinline__ SzOffsets(bool act, int wn, int lane) {
     const int c = lane & 15;
 #pragma unroll
-    for (int tt = 0; tt < TW; ++tt) {
+    for (int nt = 0; nt < NT; ++nt) {
+      const int tt = Wt::tile_of(nt, lane);
       int r, u;
       if (act && TW % 2 == 1) {  // waves pair up: wn < NWN / 2 gate, the others up
         constexpr int kHalfWaves = BN / (32 * TW);
@@ -156,22 +246,34 @@ struct SzOffsets {
         r = p >= BN / 2;
         u = p - r * (BN / 2);
       }
-      s[tt] = static_cast<uint32_t>(BN * r + 2 * u + 2 * (c & ~1));
-      z[tt] = static_cast<uint32_t>(kSzZeroBase + 16 * sz_zero_chunks<BN>() * r + 4 * (u >> 3) + 4 * (c >> 3));
+      s[nt] = static_cast<uint32_t>(BN * r + 2 * u + 2 * (c & ~1));
+      z[nt] = static_cast<uint32_t>(kSzZeroBase + 16 * sz_zero_chunks<BN>() * r + 4 * (u >> 3) + 4 * (c >> 3));
     }
   }
 };
 
-// The scale pair and zero words of the lane's columns in one group's stage.  Read right
-// after the batch barrier, ahead of the next batch's load issue, so that their latency is
-// not on the path into the group's first dequant.
-template <int TW, int BN>
-__device__ __forceinline__ void read_group_scales(GroupScales<TW>& gs, const uint8_t* sz, const SzOffsets<TW, BN>& szo) {
+// The scale pair and zero words of the lane's columns in one group's stage.
+template <class Wt, int BN>
+__device__ __forceinline__ void read_group_scales(GroupScales<Wt::NT>& gs, const uint8_t* sz,
+                                                  const SzOffsets<Wt, BN>& szo) {
 #pragma unroll
-  for (int tt = 0; tt < TW; ++tt) {
-    gs.s[tt] = *reinterpret_cast<const uint32_t*>(sz + szo.s[tt]);
-    gs.zw[tt] = *reinterpret_cast<const uint32_t*>(sz + szo.z[tt]);
+  for (int nt = 0; nt < Wt::NT; ++nt) {
+    gs.s[nt] = *reinterpret_cast<const uint32_t*>(sz + szo.s[nt]);
+    gs.zw[nt] = *reinterpret_cast<const uint32_t*>(sz + szo.z[nt]);
   }
+}
+
+// The wide form's A fragments: lane byte offset, within an activation stage, of its fragment of
+// matrix step 0.  Step s is at o ^ (its chunk << 4): the chunk of a step and the lane's own
+// chunk bits are disjoint, and the swizzle is an exclusive or.
+__device__ __forceinline__ uint32_t wide_a_offset(int lane) {
+  return static_cast<uint32_t>((lane & 31) * kARowBytes + (((2 * (lane >> 5)) ^ (lane & 15)) << 4));
+}
+
+// A fragment of row block mt at matrix step s (32-row step s / 2, K half s % 2).
+__device__ __forceinline__ bf16x8_t read_wide_a(const uint8_t* stage, uint32_t o, int s, int mt) {
+  const uint32_t chunk = 4u * (s / 2) + s % 2;
+  return *reinterpret_cast<const bf16x8_t*>(stage + (o ^ (chunk << 4)) + mt * 32 * kARowBytes);
 }
 
 // Lane byte offsets, within an activation stage, of the wave's first fragment of each of a
@@ -201,8 +303,9 @@ struct AOffsets {
 // and 64-row wave tiles (the LDS reads, then one MFMA and one to three VALU at a time)
 // 1-7 % slower at M = 48 - 256.
 template <int WM, int TW>
-__device__ __forceinline__ void mma_group(f32x4_t (&acc)[WM][TW], const uint8_t* stage, const AOffsets<WM>& ao,
-                                          const BGroup<TW>& b, const NibbleConsts& nib, int lane) {
+__device__ __forceinline__ void mma_group(WaveTile<WM, TW, false>& wt, const uint8_t* stage, const AOffsets<WM>& ao,
+                                          const BGroup<WaveTile<WM, TW, false>>& b, const NibbleConsts& nib, int lane) {
+  auto& acc = wt.acc;
   const int zshift = awq_shift(lane & 7);
   TileScale ts[TW];
 #pragma unroll
@@ -313,7 +416,7 @@ __device__ __forceinline__ void static_for(F&& f) {
 // bf16 layer outputs, as in the reference's two steps) and stores the rounded chunk.  Every
 // wave of the workgroup passes the barriers, those without columns too.
 template <int WM, int TW, int NWG, int S, int kStage, class StageFn>
-__device__ __forceinline__ void cross_silu_epilogue(const f32x4_t (&acc)[WM][TW], StageFn stage, const TileOut& o,
+__device__ __forceinline__ void cross_silu_epilogue(const WaveTile<WM, TW, false>& wt, StageFn stage, const TileOut& o,
                                                     int wave_in, int lane) {
   constexpr int WR = 16 * WM;
   constexpr int CPR = 2 * TW;  // 16-byte chunks per row
@@ -355,7 +458,7 @@ __device__ __forceinline__ void cross_silu_epilogue(const f32x4_t (&acc)[WM][TW]
             const int r = 16 * ml + 4 * (lane >> 4) + i;
             const int c = 16 * t + (lane & 15);
             const int off = r * PITCH + ((((c >> 3) + r) % CPR) << 4) + ((c & 7) << 1);
-            *reinterpret_cast<uint16_t*>(own + off) = f32_to_bf16_bits(acc[part * MP + ml][t][i]);
+            *reinterpret_cast<uint16_t*>(own + off) = f32_to_bf16_bits(wt.acc[part * MP + ml][t][i]);
           }
     }
     __syncthreads();
@@ -384,9 +487,10 @@ __device__ __forceinline__ void cross_silu_epilogue(const f32x4_t (&acc)[WM][TW]
 // between workgroups (split > 1) and the epilogue.  stage(i), i < S, is LDS region i of
 // kStage bytes; all of them are free here.  Every wave of the workgroup calls this (the
 // barriers count them all); only slice 0 holds results afterwards.
-template <int WM, int TW, int NWG, int WK, int S, int kStage, class StageFn>
-__device__ __forceinline__ void finish_tile(f32x4_t (&acc)[WM][TW], StageFn stage, int* is_last_lds,
+template <int WM, int TW, bool WIDE, int NWG, int WK, int S, int kStage, class StageFn>
+__device__ __forceinline__ void finish_tile(WaveTile<WM, TW, WIDE>& wt, StageFn stage, int* is_last_lds,
                                             const TileOut& o, int wave_in, int wk, int lane) {
+  typedef WaveTile<WM, TW, WIDE> Wt;
   if constexpr (WK > 1) {
     // Sum the slices' tiles in slice order: slices 1 .. WK - 1 park theirs in the stages
     // (lane-major fragments, 1 KiB each), slice 0 adds them to its own.  Parking slot
@@ -408,7 +512,7 @@ __device__ __forceinline__ void finish_tile(f32x4_t (&acc)[WM][TW], StageFn stag
       constexpr int k2 = decltype(k2_tag)::value;
       static_for<kFragsW>([&](auto f_tag) {
         constexpr int f = decltype(f_tag)::value;
-        *slot_ptr(std::integral_constant<int, (k2 - 1) * kFragsW + f>{}) = acc[f / TW][f % TW];
+        *slot_ptr(std::integral_constant<int, (k2 - 1) * kFragsW + f>{}) = wt.get(f);
       });
     };
     if (wk > 0) {
@@ -423,7 +527,7 @@ __device__ __forceinline__ void finish_tile(f32x4_t (&acc)[WM][TW], StageFn stag
         constexpr int k2 = decltype(i_tag)::value + 1;
         static_for<kFragsW>([&](auto f_tag) {
           constexpr int f = decltype(f_tag)::value;
-          acc[f / TW][f % TW] += *slot_ptr(std::integral_constant<int, (k2 - 1) * kFragsW + f>{});
+          wt.set(f, wt.get(f) + *slot_ptr(std::integral_constant<int, (k2 - 1) * kFragsW + f>{}));
         });
       });
     }
@@ -451,7 +555,7 @@ __device__ __forceinline__ void finish_tile(f32x4_t (&acc)[WM][TW], StageFn stag
     };
     if (wk == 0) {
 #pragma unroll
-      for (int f = 0; f < kFrags; ++f) store_fragment(rp, frag_off(sidx, f), acc[f / TW][f % TW]);
+      for (int f = 0; f < kFrags; ++f) store_fragment(rp, frag_off(sidx, f), wt.get(f));
     }
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
@@ -466,7 +570,7 @@ __device__ __forceinline__ void finish_tile(f32x4_t (&acc)[WM][TW], StageFn stag
       for (int sp = 0; sp < split; ++sp) {
         if (sp == sidx) {
 #pragma unroll
-          for (int f = 0; f < KC; ++f) tot[f] += acc[(c + f) / TW][(c + f) % TW];
+          for (int f = 0; f < KC; ++f) tot[f] += wt.get(c + f);
         } else {
           f32x4_t part[KC];
 #pragma unroll
@@ -476,14 +580,14 @@ __device__ __forceinline__ void finish_tile(f32x4_t (&acc)[WM][TW], StageFn stag
         }
       }
 #pragma unroll
-      for (int f = 0; f < KC; ++f) acc[(c + f) / TW][(c + f) % TW] = tot[f];
+      for (int f = 0; f < KC; ++f) wt.set(c + f, tot[f]);
     }
     if (threadIdx.x == 0) rearm(&counters[tile]);
   }
 
   if constexpr (TW % 2 == 1) {
     if (o.act) {  // uniform: waves paired along N (WK == 1)
-      cross_silu_epilogue<WM, TW, NWG, S, kStage>(acc, stage, o, wave_in, lane);
+      cross_silu_epilogue<WM, TW, NWG, S, kStage>(wt, stage, o, wave_in, lane);
       return;
     }
   }
@@ -550,7 +654,7 @@ __device__ __forceinline__ void finish_tile(f32x4_t (&acc)[WM][TW], StageFn stag
             const int r = 16 * ml + 4 * (lane >> 4) + i;
             const int c = 16 * t + (lane & 15);
             const int off = r * PITCH + ((((c >> 3) + r) % CPR) << 4) + ((c & 7) << 1);
-            *reinterpret_cast<uint16_t*>(ep + off) = f32_to_bf16_bits(acc[part * MP + ml][t][i]);
+            *reinterpret_cast<uint16_t*>(ep + off) = f32_to_bf16_bits(wt.acc[part * MP + ml][t][i]);
           }
       __builtin_amdgcn_s_waitcnt(0);
       __builtin_amdgcn_wave_barrier();
@@ -574,43 +678,69 @@ __device__ __forceinline__ void finish_tile(f32x4_t (&acc)[WM][TW], StageFn stag
   } else if (!o.act) {
     constexpr int TP0 = TW / kParts;
     constexpr int TP = TP0 & -TP0;  // tiles per pass: a power of two, so that rows are whole lane groups
+    constexpr int NB = 16 * TP / Wt::kCols;  // column blocks per pass
+    static_assert(NB > 0, "passes of whole column blocks");
     constexpr int CPR = 2 * TP;     // 16-byte chunks per row
     constexpr int PITCH = 16 * CPR;
 #pragma unroll
     for (int part = 0; part < TW / TP; ++part) {
 #pragma unroll
-      for (int mt = 0; mt < WM; ++mt)
+      for (int mt = 0; mt < Wt::MT; ++mt)
 #pragma unroll
-        for (int t = 0; t < TP; ++t)
+        for (int nt = 0; nt < NB; ++nt)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int r = 16 * mt + 4 * (lane >> 4) + i;
-            const int c = 16 * t + (lane & 15);
+          for (int e = 0; e < 4 * Wt::Q; ++e) {
+            const int r = Wt::row(mt, e / 4, e % 4, lane);
+            const int c = Wt::col(nt, lane);
             const int off = r * PITCH + (((c >> 3) ^ (r % CPR)) << 4) + ((c & 7) << 1);
-            *reinterpret_cast<uint16_t*>(ep + off) = f32_to_bf16_bits(acc[mt][part * TP + t][i]);
+            *reinterpret_cast<uint16_t*>(ep + off) = f32_to_bf16_bits(wt.acc[mt][part * NB + nt][e]);
           }
       store_rows(std::integral_constant<int, CPR>{}, o.col_w + 16 * TP * part);
     }
-  } else if constexpr (TW % 2 == 0) {  // the fused product pairs the two halves of a wave's tiles
-    constexpr int H = TW / 2;
-    constexpr int TP0 = (H % kParts == 0) ? H / kParts : H;
-    constexpr int TP = TP0 & -TP0;  // gate tiles per pass (a power of two)
-    constexpr int NP = H / TP;
+  } else if constexpr (Wt::kWide && TW == 2) {
+    // One column block: gate columns in the lanes with lane / 16 even, their up columns 16
+    // lanes on.  Half of each lane's values change places, so that every lane holds both
+    // operands of half of the rows: gate lanes those of fragments 0 and 1, up lanes of 2, 3.
+    constexpr int CPR = 2;
+    constexpr int PITCH = 16 * CPR;
+    const bool up = (lane & 16) != 0;
+#pragma unroll
+    for (int mt = 0; mt < Wt::MT; ++mt)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        // swap the odd lane rows of fragment value e with the even ones of e + 8 (the empty asm
+        // keeps both in VGPRs: the swap takes no accumulation registers)
+        uint32_t lo = __float_as_uint(wt.acc[mt][0][e]), hi = __float_as_uint(wt.acc[mt][0][e + 8]);
+        asm volatile("" : "+v"(lo), "+v"(hi));
+        const auto gu = __builtin_amdgcn_permlane16_swap(lo, hi, false, false);
+        const int r = Wt::row(mt, e / 4 + (up ? 2 : 0), e % 4, lane);
+        const int c = lane & 15;
+        const int off = r * PITCH + (((c >> 3) ^ (r % CPR)) << 4) + ((c & 7) << 1);
+        *reinterpret_cast<uint16_t*>(ep + off) = f32_to_bf16_bits(silu_mul_of_bf16(__uint_as_float(gu[0]), __uint_as_float(gu[1])));
+      }
+    store_rows(std::integral_constant<int, CPR>{}, o.col_w);
+  } else if constexpr (TW % 2 == 0) {  // the fused product pairs the two halves of a wave's blocks
+    constexpr int H = Wt::NT / 2;                // gate blocks
+    constexpr int HT = TW / 2;                   // gate tiles
+    constexpr int TP0 = HT % kParts == 0 && HT / kParts * 16 >= Wt::kCols ? HT / kParts : HT;
+    constexpr int TP = TP0 & -TP0;               // gate tiles per pass (a power of two)
+    constexpr int NB = 16 * TP / Wt::kCols;      // gate blocks per pass
     constexpr int CPR = 2 * TP;
     constexpr int PITCH = 16 * CPR;
+    static_assert(WR * PITCH <= kRegion, "a pass fits the wave's region");
 #pragma unroll
-    for (int part = 0; part < NP; ++part) {
+    for (int part = 0; part < H / NB; ++part) {
 #pragma unroll
-      for (int mt = 0; mt < WM; ++mt)
+      for (int mt = 0; mt < Wt::MT; ++mt)
 #pragma unroll
-        for (int t = 0; t < TP; ++t)
+        for (int nt = 0; nt < NB; ++nt)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int r = 16 * mt + 4 * (lane >> 4) + i;
-            const int c = 16 * t + (lane & 15);
+          for (int e = 0; e < 4 * Wt::Q; ++e) {
+            const int r = Wt::row(mt, e / 4, e % 4, lane);
+            const int c = Wt::col(nt, lane);
             const int off = r * PITCH + (((c >> 3) ^ (r % CPR)) << 4) + ((c & 7) << 1);
-            const int tt = part * TP + t;
-            *reinterpret_cast<uint16_t*>(ep + off) = f32_to_bf16_bits(silu_mul_of_bf16(acc[mt][tt][i], acc[mt][tt + H][i]));
+            const int g = part * NB + nt;
+            *reinterpret_cast<uint16_t*>(ep + off) = f32_to_bf16_bits(silu_mul_of_bf16(wt.acc[mt][g][e], wt.acc[mt][g + H][e]));
           }
       store_rows(std::integral_constant<int, CPR>{}, o.col_w + 16 * TP * part);
     }

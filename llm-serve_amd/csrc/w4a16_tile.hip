@@ -38,8 +38,6 @@
 
 namespace w4a16 {
 
-typedef __attribute__((address_space(3))) void lds_void_t;
-
 // Issue the direct-to-LDS loads of activation rows [row0, row0 + BM) x group g into `stage`
 // (NW waves, NI instructions each).  Instruction i of wave w fills rows 4 (NW i + w) .. +3
 // (1 KiB); lane -> (row, physical chunk).  When the BM / 4 row quads do not split evenly over
@@ -49,7 +47,7 @@ typedef __attribute__((address_space(3))) void lds_void_t;
 // offset is the instruction's scalar offset, the lane's part the same for every group, and
 // their sum stays inside the activations (rows past M read row M - 1).
 template <int NI, int NW, int BM>
-__device__ __forceinline__ void issue_a_stage(__amdgpu_buffer_rsrc_t rx, uint8_t* stage, uint8_t* spare, int row0,
+__device__ __forceinline__ void issue_a_stage(__amdgpu_buffer_rsrc_t rx, lds_u8_t* stage, lds_u8_t* spare, int row0,
                                               int M, int K, int g, int wave, int lane) {
   const int p = lane & 15;
 #pragma unroll
@@ -153,14 +151,12 @@ __global__ __launch_bounds__(64 * NWM * NWN * WK, OCC) void tile_kernel(const ui
   // The workgroup's two column ranges of BN / 2 (scale and zero staging).
   const int cs0 = act ? nbk * (BN / 2) : nbk * BN;
   const int cs1 = act ? cs0 + up_tiles * kTileCols : cs0 + BN / 2;
-  const SzOffsets<TW, BN> szo(act, wn, lane);
+  typedef WaveTile<WM, TW, false> Wt;
+  const SzOffsets<Wt, BN> szo(act, wn, lane);
   const AOffsets<WM> ao(wm, lane);
 
-  f32x4_t acc[WM][TW];
-#pragma unroll
-  for (int mt = 0; mt < WM; ++mt)
-#pragma unroll
-    for (int tt = 0; tt < TW; ++tt) acc[mt][tt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  Wt wt;
+  wt.clear();
 
   // Batched pipeline over the workgroup's groups (item i = group g_begin + i).  Items travel
   // in batches of P: batch b (items b .. b + P - 1) lives in LDS stages P h .. P h + P - 1,
@@ -179,23 +175,23 @@ __global__ __launch_bounds__(64 * NWM * NWN * WK, OCC) void tile_kernel(const ui
                       make_buffer(qzeros, static_cast<uint32_t>(G) * (N / 8) * 4u)};
   constexpr int kWaitAll = 0x0F70;  // vmcnt(0); expcnt and lgkmcnt not waited for
   const int n_items = g_end - g_begin;
-  BGroup<TW> ring[2 * PW];
+  BGroup<Wt> ring[2 * PW];
   // A prefetch past the workgroup's last item reloads that item's group (never consumed);
   // ranges are never empty (split <= K / 128).
   auto group_of = [&](int item) { return g_begin + (item < n_items ? item : n_items - 1); };
   auto issue = [&](int half, int b) {  // batch starting at item b into half `half`
 #pragma unroll
     for (int q = 0; q < P; ++q) {
-      issue_a_stage<NI, NW, BM>(rx, stage(half * P + q), spare, row0, M, K, group_of(b + q), wave, lane);
+      issue_a_stage<NI, NW, BM>(rx, (lds_u8_t*)stage(half * P + q), (lds_u8_t*)spare, row0, M, K, group_of(b + q), wave, lane);
       // the group's scale and zero instructions go to waves 2q and 2q + 1 (mod NW)
       if (kStageSZ && (wave == (2 * q) % NW || wave == (2 * q + 1) % NW))
-        issue_sz_stage<BN>(bsrc, sz_stage[kStageSZ ? half * P + q : 0], group_of(b + q), N, cs0, cs1,
+        issue_sz_stage<BN>(bsrc, (lds_u8_t*)sz_stage[kStageSZ ? half * P + q : 0], group_of(b + q), N, cs0, cs1,
                            wave == (2 * q) % NW ? 0 : 1, lane);
     }
 #pragma unroll
     for (int j = 0; j < PW; ++j) {
       const int item = b + wk + WK * j;
-      load_b_group<TW, !kStageSZ>(ring[half * PW + j], bsrc, group_of(item), active, N, t0, dt, lane);
+      load_b_group<Wt, !kStageSZ>(ring[half * PW + j], bsrc, group_of(item), active, N, t0, dt, lane);
     }
   };
   issue(0, 0);
@@ -213,7 +209,7 @@ __global__ __launch_bounds__(64 * NWM * NWN * WK, OCC) void tile_kernel(const ui
         if constexpr (kStageSZ) {
 #pragma unroll
           for (int j = 0; j < PW; ++j)  // the wave's groups of the batch: items b + wk + WK j
-            read_group_scales<TW, BN>(ring[h * PW + j].sc, sz_stage[h * P + wk + WK * j], szo);
+            read_group_scales<Wt, BN>(ring[h * PW + j].sc, sz_stage[h * P + wk + WK * j], szo);
           __builtin_amdgcn_sched_barrier(0);
         }
         // nothing past the last item (the full wait at the next batch would wait for it)
@@ -223,7 +219,7 @@ __global__ __launch_bounds__(64 * NWM * NWN * WK, OCC) void tile_kernel(const ui
         for (int q = 0; q < P; ++q) {
           // q is a constant, so the stage is a known LDS object; the slice test is uniform
           if (q % WK == wk && b + q < n_items && active)
-            mma_group<WM, TW>(acc, stage(h * P + q), ao, ring[h * PW + q / WK], nib, lane);
+            mma_group<WM, TW>(wt, stage(h * P + q), ao, ring[h * PW + q / WK], nib, lane);
         }
       }
     }
@@ -233,8 +229,199 @@ __global__ __launch_bounds__(64 * NWM * NWN * WK, OCC) void tile_kernel(const ui
 
   TileOut out{y, res, partials, counters, M, N, n_out, split, sidx, mbk * n_blocks + nbk, m_blocks * n_blocks,
               row0 + wm * 16 * WM, col_w, act, active};
-  finish_tile<WM, TW, NWG, WK, S, kStage>(acc, stage, &is_last, out, wave_in, wk, lane);
+  finish_tile<WM, TW, false, NWG, WK, S, kStage>(wt, stage, &is_last, out, wave_in, wk, lane);
 }
+
+// The kernel of 64- and 96-row tiles of eight 32-column waves over all of K: tile_kernel's tiles
+// and operand staging, on 32x32x16 MFMAs and with the K loop rolled over the group boundary.
+//
+// Why.  At these heights a weight serves few rows, so issue and waits bound the loop and not
+// the matrix pipe.  In tile_kernel every group begins behind its barrier with an LDS read, the
+// scale set-up and a dequant in front of its first MFMA, in all waves at once.  Here, while a
+// matrix step's MFMAs run, each A register is refilled for kAhead steps later as soon as its
+// MFMA has issued and the next step's weights are dequantized; the last steps of a group do so
+// for the first steps of the next one.  The group's one wait and barrier come kAhead steps
+// before its end, so every wave leaves the barrier with MFMAs to issue.  Measured on MI355X:
+// gate_up 4096 x 24576 at M = 150 on 96 x 256 tiles 43.5 against 47.0 us; two decoder layers'
+// graph at M = 150 / 170 / 189 247.6 / 256.1 / 257.4 against 262.1 / 274.0 / 275.9 us.
+//
+// Where not.  Taller tiles run at the power limit and take the narrow form (see WaveTile): 1 -
+// 5 % slower here, and 64-column waves spill.  Tiles whose waves split K run 3 to 16 batches a
+// launch: back to back they gained 0 - 10 %, but between other kernels, as a model runs them,
+// they lost (two layers' graph at M = 64 / 96 / 256 / 512 1 / 3 / 3 / 2 % slower).  A ring of
+// four weight slots, with waits that leave the newest in flight, was 0 - 5 % slower than two.
+template <int WM, int NWN, int OCC>
+__global__ __launch_bounds__(64 * NWN, OCC) void roll_kernel(const uint16_t* __restrict__ x,
+                                                             const uint32_t* __restrict__ packed,
+                                                             const uint32_t* __restrict__ qzeros,
+                                                             const uint16_t* __restrict__ scales, uint16_t* y,
+                                                             const uint16_t* res, float* __restrict__ partials,
+                                                             int* __restrict__ counters, int M, int K, int N,
+                                                             int split, int m_blocks, int n_blocks, int up_tiles) {
+  constexpr int TW = 2;
+  typedef WaveTile<WM, TW, true> Wt;
+  constexpr int BM = 16 * WM;
+  constexpr int BN = 16 * TW * NWN;
+  constexpr int NI = BM / 4 / NWN;  // activation-stage instructions per wave and group
+  static_assert(NI * NWN * 4 == BM, "the row quads split evenly over the waves");
+  constexpr int kStage = BM * kARowBytes;
+  // One LDS object per stage: the compiler then knows that a direct-to-LDS load into one does
+  // not alias the reads of the other, and does not wait for the loads just issued (the group
+  // after next) before reading the next one.
+  __shared__ __attribute__((aligned(1024))) uint8_t stage0[kStage];
+  __shared__ __attribute__((aligned(1024))) uint8_t stage1[kStage];
+  __shared__ __attribute__((aligned(16))) uint8_t sz0[kSzStageBytes];  // scales and zero words
+  __shared__ __attribute__((aligned(16))) uint8_t sz1[kSzStageBytes];
+  __shared__ int is_last;
+
+  const int lane = threadIdx.x & 63;
+  const int wave = wave_id();  // column slice
+  const int G = K / kGroup;
+
+  const TileCoord tc = tile_coord(blockIdx.x, m_blocks, n_blocks, split);
+  const int sidx = tc.sidx, mbk = tc.mbk, nbk = tc.nbk;
+  const int g_begin = (G * sidx) / split;
+  const int n_groups = (G * (sidx + 1)) / split - g_begin;  // never 0 (split <= K / 128)
+  const int row0 = mbk * BM;
+  // Plain: the wave computes output columns [col_w, col_w + 32) = layout tiles t0, t0 + 1.
+  // Fused SiLU(gate) * up (up_tiles = N / 32): output columns [col_w, col_w + 16) of the
+  // [M, N / 2] result, from gate tile t0 and up tile t0 + up_tiles.
+  const bool act = up_tiles != 0;
+  const int n_out = act ? N / 2 : N;
+  const int col_w = act ? nbk * (BN / 2) + 8 * TW * wave : nbk * BN + 16 * TW * wave;
+  const int t0 = col_w / kTileCols;
+  const int dt = act ? up_tiles - TW / 2 : 0;
+  const bool active = col_w < n_out;  // wave-uniform (n_out % 64 == 0): the last n-block may be partly past it
+  // The workgroup's two column ranges of BN / 2 (scale and zero staging).
+  const int cs0 = act ? nbk * (BN / 2) : nbk * BN;
+  const int cs1 = act ? cs0 + up_tiles * kTileCols : cs0 + BN / 2;
+  const SzOffsets<Wt, BN> szo(act, wave, lane);
+  const uint32_t ao = wide_a_offset(lane);
+
+  Wt wt;
+  wt.clear();
+
+  // Group g lives in LDS stage and register slot g % 2 (counted from the workgroup's first), its
+  // loads issued one group of compute ahead.  Past group g's barrier, kAhead steps before its
+  // end, group g + 1 has landed and every wave has read all of group g, so the loads of group
+  // g + 2 go into its stage, and at the last step, once the slot's last word is dequantized,
+  // into its registers.  The wait is for all loads (direct-to-LDS loads may complete out of
+  // order with the register loads issued after them).
+  const NibbleConsts nib = nibble_consts();
+  const __amdgpu_buffer_rsrc_t rx = make_buffer(x, static_cast<uint32_t>(M) * K * 2u);
+  const BSources bsrc{make_buffer(packed, static_cast<uint32_t>(K) * (N / 2)),
+                      make_buffer(scales, static_cast<uint32_t>(G) * N * 2u),
+                      make_buffer(qzeros, static_cast<uint32_t>(G) * (N / 8) * 4u)};
+  constexpr int kWaitAll = 0x0F70;  // vmcnt(0); expcnt and lgkmcnt not waited for
+  constexpr int kSteps = Wt::kSteps;
+  constexpr int kAhead = 2;  // steps of A fragments held: a step's two or three MFMAs do not cover an LDS read
+  BGroup<Wt> ring[2];
+  auto issue_lds = [&](auto slot_tag, int g) {  // activations, scales and zeros of group g
+    constexpr int slot = decltype(slot_tag)::value;
+    issue_a_stage<NI, NWN, BM>(rx, (lds_u8_t*)(slot ? stage1 : stage0), nullptr, row0, M, K, g_begin + g, wave, lane);
+    if (wave < 2) issue_sz_stage<BN>(bsrc, (lds_u8_t*)(slot ? sz1 : sz0), g_begin + g, N, cs0, cs1, wave, lane);
+  };
+  auto issue_w = [&](auto slot_tag, int g) {  // the wave's weights of group g
+    load_b_group<Wt, false>(ring[decltype(slot_tag)::value], bsrc, g_begin + g, active, N, t0, dt, lane);
+  };
+  const int zshift = awq_shift(lane & 7);
+  TileScale ts;
+  GroupScales<1> gs;  // raw scale and zero of the group that ts is made for next
+  bf16x8_t a[kAhead][Wt::MT];
+  bf16x8_t bf[2];
+  auto read_scales = [&](auto slot_tag) {
+    read_group_scales<Wt, BN>(gs, decltype(slot_tag)::value ? sz1 : sz0, szo);
+  };
+  auto make_scale = [&] { ts = make_tile_scale(gs.s[0], (gs.zw[0] >> zshift) & 0xFu, lane); };
+
+  // Group g in slot h, whose first kAhead steps of A and first step of weights are in registers.
+  auto compute_group = [&](auto slot_tag, int g) {
+    constexpr int h = decltype(slot_tag)::value;
+    const uint8_t* cur = h ? stage1 : stage0;
+    const uint8_t* nxt = h ? stage0 : stage1;
+    ScaledStep sd;
+    static_for<kSteps>([&](auto s_tag) {
+      constexpr int s = decltype(s_tag)::value;
+      if constexpr (s == kSteps - kAhead) {
+        // Group g + 1 has landed.  (Waited for on the last group too, where nothing is in
+        // flight: behind the branch, the compiler would wait again for the ring's loads, and
+        // with them for the ones just issued.)
+        __builtin_amdgcn_s_waitcnt(kWaitAll);
+        if (g + 1 < n_groups) __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);
+        read_scales(std::integral_constant<int, 1 - h>{});  // past the last group: stale words, not used
+        if (g + 2 < n_groups) issue_lds(slot_tag, g + 2);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if constexpr (s == kSteps - 1) {
+        make_scale();
+        if (g + 2 < n_groups) issue_w(slot_tag, g + 2);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      static_for<Wt::MT>([&](auto mt_tag) {
+        constexpr int mt = decltype(mt_tag)::value;
+        constexpr int sr = s + kAhead;
+        wt.acc[mt][0] = Wt::mfma(a[s % kAhead][mt], bf[s & 1], wt.acc[mt][0]);
+        a[s % kAhead][mt] = read_wide_a(sr < kSteps ? cur : nxt, ao, sr % kSteps, mt);
+        // The next step's weights: unpacked and scaled beside the first row block's MFMA, and
+        // rounded beside the last one's, which then does not wait for the scaling.
+        if constexpr (mt == 0) sd = dequant_scale(s + 1 < kSteps ? ring[h].word(0, s + 1) : ring[1 - h].word(0, 0), ts, nib);
+        if constexpr (mt == Wt::MT - 1) bf[(s + 1) & 1] = dequant_pack(sd);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    });
+  };
+
+  constexpr std::integral_constant<int, 0> k0{};
+  constexpr std::integral_constant<int, 1> k1{};
+  issue_lds(k0, 0);
+  issue_w(k0, 0);
+  __builtin_amdgcn_s_waitcnt(kWaitAll);
+  __syncthreads();
+  __builtin_amdgcn_sched_barrier(0);
+  if (n_groups > 1) {
+    issue_lds(k1, 1);
+    issue_w(k1, 1);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  if (active) {
+    read_scales(k0);
+    make_scale();
+    static_for<kAhead>([&](auto s_tag) {
+      constexpr int s = decltype(s_tag)::value;
+#pragma unroll
+      for (int mt = 0; mt < Wt::MT; ++mt) a[s][mt] = read_wide_a(stage0, ao, s, mt);
+    });
+    bf[0] = dequant_step(ring[0].word(0, 0), ts, nib);
+    // Two groups per trip, so that the slot is a constant, and no branch around either: one
+    // that could skip the odd group carries the even one's loads into a wait at the top.
+    int g = 0;
+    for (; g + 2 <= n_groups; g += 2) {
+      compute_group(k0, g);
+      compute_group(k1, g + 1);
+    }
+    if (g < n_groups) compute_group(k0, g);
+  } else {  // columns past N: the wave only takes its part in the loads and barriers
+    for (int g = 0; g + 1 < n_groups; ++g) {
+      __builtin_amdgcn_s_waitcnt(kWaitAll);
+      __syncthreads();
+      if (g + 2 < n_groups) {
+        if (g & 1) issue_lds(k1, g + 2);
+        else issue_lds(k0, g + 2);
+      }
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+
+  auto stage = [&](int st) -> uint8_t* { return st ? stage1 : stage0; };
+  TileOut out{y, res, partials, counters, M, N, n_out, split, sidx, mbk * n_blocks + nbk, m_blocks * n_blocks,
+              row0, col_w, act, active};
+  finish_tile<WM, TW, true, NWN, 1, 2, kStage>(wt, stage, &is_last, out, wave, 0, lane);
+}
+
+// Which compiled tiles take roll_kernel (see there).
+constexpr bool tile_rolls(int wm, int tw, int nwm, int wk) { return tw == 2 && wm <= 6 && nwm == 1 && wk == 1; }
 
 template <int WM, int TW, int NWM, int NWN, int OCC, int WK>
 static hipError_t launch_tile_t(const uint16_t* x, const uint32_t* packed, const uint32_t* qzeros,
@@ -245,8 +432,12 @@ static hipError_t launch_tile_t(const uint16_t* x, const uint32_t* packed, const
   const int m_blocks = (M + BM - 1) / BM;
   const int n_blocks = (N + BN - 1) / BN;
   const unsigned grid = static_cast<unsigned>(m_blocks * n_blocks * split);
-  tile_kernel<WM, TW, NWM, NWN, OCC, WK><<<grid, 64 * NWM * NWN * WK, 0, stream>>>(
-      x, packed, qzeros, scales, y, res, partials, counters, M, K, N, split, m_blocks, n_blocks, up_tiles);
+  if constexpr (tile_rolls(WM, TW, NWM, WK))
+    roll_kernel<WM, NWN, OCC><<<grid, 64 * NWN, 0, stream>>>(
+        x, packed, qzeros, scales, y, res, partials, counters, M, K, N, split, m_blocks, n_blocks, up_tiles);
+  else
+    tile_kernel<WM, TW, NWM, NWN, OCC, WK><<<grid, 64 * NWM * NWN * WK, 0, stream>>>(
+        x, packed, qzeros, scales, y, res, partials, counters, M, K, N, split, m_blocks, n_blocks, up_tiles);
   return hipGetLastError();
 }
 

@@ -11,7 +11,8 @@ import pytest
 import torch
 
 from awq_helpers import (GEMM_REL_TOL, QWEN3_SHAPES, awq_mod, bf16_from_bits, bits_of, decode_config_accepted,
-                         golden_cases, pkg, random_awq_gpu, random_x_gpu, rel_err, to_gpu, assert_gemm_close)
+                         golden_cases, pkg, random_awq_gpu, random_x_gpu, rel_err, to_gpu, assert_gemm_close,
+                         assert_silu_two_step)
 from oracle import awq_oracle as ora
 
 pytestmark = pytest.mark.gpu
@@ -133,6 +134,37 @@ def test_every_tile_configuration(gpu_lib, m, n):
         assert_gemm_close(y, want, (wm, shape, occ, split))
         if ws_bytes:  # arrival counters (the first 64 KiB) are re-armed to zero
             assert int(torch.count_nonzero(ws[:65536])) == 0
+
+
+@pytest.mark.parametrize("groups", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("wm", [4, 6])
+def test_rolled_tiles_at_group_and_tile_edges(gpu_lib, groups, wm):
+    """The 64- and 96-row tiles of eight 32-column waves, whose K loop rolls over the group
+    boundary: one to five groups (odd and even, the loop's trips and its tail) with K whole and
+    split, row blocks that end on, before and after M, and column blocks with whole waves past N
+    (N = 64, 320), plain and -- where N % 128 == 0 -- fused."""
+    k = 128 * groups
+    awq = awq_mod()
+    for n in (64, 128, 320, 640):
+        p = ora.make_problem(seed=groups * 1000 + n, m=2 * 16 * wm + 1, k=k, n=n)
+        t = to_gpu(p)
+        packed = awq.repack_awq_qweight(t["qweight"])
+        want = torch.from_numpy(ora.awq_linear_ref(p["x_bits"], p["qweight"], p["qzeros"], p["scales_bits"], 128)).cuda()
+        w = awq.dequantize_awq_gemm(t["qweight"], t["qzeros"], t["scales"], group_size=128).float()
+        for m in (1, 16 * wm - 1, 16 * wm, 16 * wm + 1, 2 * 16 * wm + 1):
+            for split in (1, 2):
+                if split > groups:
+                    continue
+                ws = torch.zeros(max(gpu_lib.workspace_bytes_config(m, n, 2, wm, split), 1), dtype=torch.uint8, device="cuda")
+                x = t["x"][:m].contiguous()
+                y = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+                gpu_lib.gemm_config(x, packed, t["qzeros"], t["scales"], y, k, n, 2, wm, 2, split, ws, p2=3)
+                assert_gemm_close(y, want[:m], (wm, k, n, m, split))
+                if n % 128 == 0:
+                    f = torch.full((m, n // 2), float("nan"), dtype=torch.bfloat16, device="cuda")
+                    gpu_lib.gemm_config(x, packed, t["qzeros"], t["scales"], f, k, n, 2, wm, 2, split, ws, p2=3,
+                                        silu_mul=True)
+                    assert_silu_two_step(f, x, w, (wm, k, n, m, split))
 
 
 def test_scales_and_zeros_at_word_alignment(gpu_lib):
