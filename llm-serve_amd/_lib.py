@@ -98,9 +98,18 @@ class W4A16Library:
         if status != 0:
             raise W4A16Error(f"{what} failed (status {status}): {self.last_error()}")
 
-    @staticmethod
-    def _stream(t: torch.Tensor) -> int:
-        return torch.cuda.current_stream(t.device).cuda_stream
+    def _launch(self, fn, what: str, t: torch.Tensor, *args) -> None:
+        """fn(*args, stream) with t's GPU current, on its current torch stream.  Two C calls find
+        the device and the stream's raw handle; torch.cuda.device and a Stream object on every
+        call were a third of an eager call's host time."""
+        index = t.get_device()
+        if index >= 0 and torch._C._cuda_getDevice() == index:
+            status = fn(*args, torch._C._cuda_getCurrentRawStream(index))
+        else:
+            with torch.cuda.device(t.device):  # raises for a host tensor
+                status = fn(*args, torch._C._cuda_getCurrentRawStream(index))
+        if status != 0:
+            self.check(status, what)
 
     @staticmethod
     def _require_gpu(*tensors: torch.Tensor) -> None:
@@ -136,19 +145,16 @@ class W4A16Library:
         self._require_gpu(packed)
         rows, cols = packed.shape
         out = torch.empty((rows, cols * 8), dtype=torch.int32, device=packed.device)
-        with torch.cuda.device(packed.device):
-            self.check(self.dll.w4a16_unpack_int4(packed.data_ptr(), out.data_ptr(), rows, cols,
-                                                  self._stream(packed)), "w4a16_unpack_int4")
+        self._launch(self.dll.w4a16_unpack_int4, "w4a16_unpack_int4", packed, packed.data_ptr(), out.data_ptr(), rows,
+                     cols)
         return out
 
     def dequant(self, qweight, qzeros, scales, group_size: int) -> torch.Tensor:
         self._require_gpu(qweight, qzeros, scales)
         k, n = qweight.shape[0], qweight.shape[1] * 8
         out = torch.empty((k, n), dtype=torch.bfloat16, device=qweight.device)
-        with torch.cuda.device(qweight.device):
-            self.check(self.dll.w4a16_dequant(qweight.data_ptr(), qzeros.data_ptr(), scales.data_ptr(),
-                                              out.data_ptr(), k, n, group_size, self._stream(qweight)),
-                       "w4a16_dequant")
+        self._launch(self.dll.w4a16_dequant, "w4a16_dequant", qweight, qweight.data_ptr(), qzeros.data_ptr(),
+                     scales.data_ptr(), out.data_ptr(), k, n, group_size)
         return out
 
     _DTYPES = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
@@ -162,10 +168,8 @@ class W4A16Library:
         qweight = torch.empty((in_f, out_f // 8), dtype=torch.int32, device=dev)
         qzeros = torch.empty((in_f // group_size, out_f // 8), dtype=torch.int32, device=dev)
         scales = torch.empty((in_f // group_size, out_f), dtype=weight.dtype, device=dev)
-        with torch.cuda.device(dev):
-            self.check(self.dll.w4a16_quantize(weight.data_ptr(), self._DTYPES[weight.dtype], qweight.data_ptr(),
-                                               qzeros.data_ptr(), scales.data_ptr(), out_f, in_f, group_size,
-                                               self._stream(weight)), "w4a16_quantize")
+        self._launch(self.dll.w4a16_quantize, "w4a16_quantize", weight, weight.data_ptr(), self._DTYPES[weight.dtype],
+                     qweight.data_ptr(), qzeros.data_ptr(), scales.data_ptr(), out_f, in_f, group_size)
         return qweight, qzeros, scales
 
     def pack_int4(self, values: torch.Tensor) -> torch.Tensor:
@@ -173,27 +177,23 @@ class W4A16Library:
         self._require_gpu(values)
         rows, cols = values.shape
         out = torch.empty((rows, cols // 8), dtype=torch.int32, device=values.device)
-        with torch.cuda.device(values.device):
-            self.check(self.dll.w4a16_pack_int4(values.data_ptr(), out.data_ptr(), rows, cols,
-                                                self._stream(values)), "w4a16_pack_int4")
+        self._launch(self.dll.w4a16_pack_int4, "w4a16_pack_int4", values, values.data_ptr(), out.data_ptr(), rows,
+                     cols)
         return out
 
     def repack_qweight(self, qweight: torch.Tensor) -> torch.Tensor:
         self._require_gpu(qweight)
         k, n = qweight.shape[0], qweight.shape[1] * 8
         out = torch.empty((k * n // 8,), dtype=torch.int32, device=qweight.device)
-        with torch.cuda.device(qweight.device):
-            self.check(self.dll.w4a16_repack_qweight(qweight.data_ptr(), out.data_ptr(), k, n,
-                                                     self._stream(qweight)), "w4a16_repack_qweight")
+        self._launch(self.dll.w4a16_repack_qweight, "w4a16_repack_qweight", qweight, qweight.data_ptr(),
+                     out.data_ptr(), k, n)
         return out
 
     def dequant_packed(self, packed, qzeros, scales, k: int, n: int, group_size: int = 128) -> torch.Tensor:
         self._require_gpu(packed, qzeros, scales)
         out = torch.empty((k, n), dtype=torch.bfloat16, device=packed.device)
-        with torch.cuda.device(packed.device):
-            self.check(self.dll.w4a16_dequant_packed(packed.data_ptr(), qzeros.data_ptr(), scales.data_ptr(),
-                                                     out.data_ptr(), k, n, group_size, self._stream(packed)),
-                       "w4a16_dequant_packed")
+        self._launch(self.dll.w4a16_dequant_packed, "w4a16_dequant_packed", packed, packed.data_ptr(),
+                     qzeros.data_ptr(), scales.data_ptr(), out.data_ptr(), k, n, group_size)
         return out
 
     def gemm(self, x, packed, qzeros, scales, y, k: int, n: int, workspace: torch.Tensor | None,
@@ -202,10 +202,8 @@ class W4A16Library:
         m = x.shape[0]
         ws_ptr = workspace.data_ptr() if workspace is not None else None
         ws_len = workspace.numel() * workspace.element_size() if workspace is not None else 0
-        with torch.cuda.device(x.device):
-            self.check(self.dll.w4a16_gemm(x.data_ptr(), packed.data_ptr(), qzeros.data_ptr(), scales.data_ptr(),
-                                           y.data_ptr(), m, k, n, group_size, ws_ptr, ws_len, self._stream(x)),
-                       "w4a16_gemm")
+        self._launch(self.dll.w4a16_gemm, "w4a16_gemm", x, x.data_ptr(), packed.data_ptr(), qzeros.data_ptr(),
+                     scales.data_ptr(), y.data_ptr(), m, k, n, group_size, ws_ptr, ws_len)
         return y
 
     def gemm_residual(self, x, packed, qzeros, scales, residual, y, k: int, n: int,
@@ -214,11 +212,9 @@ class W4A16Library:
         m = x.shape[0]
         ws_ptr = workspace.data_ptr() if workspace is not None else None
         ws_len = workspace.numel() * workspace.element_size() if workspace is not None else 0
-        with torch.cuda.device(x.device):
-            self.check(self.dll.w4a16_gemm_residual(x.data_ptr(), packed.data_ptr(), qzeros.data_ptr(),
-                                                    scales.data_ptr(), residual.data_ptr(), y.data_ptr(), m, k, n,
-                                                    group_size, ws_ptr, ws_len, self._stream(x)),
-                       "w4a16_gemm_residual")
+        self._launch(self.dll.w4a16_gemm_residual, "w4a16_gemm_residual", x, x.data_ptr(), packed.data_ptr(),
+                     qzeros.data_ptr(), scales.data_ptr(), residual.data_ptr(), y.data_ptr(), m, k, n, group_size,
+                     ws_ptr, ws_len)
         return y
 
     def gemm_silu_mul(self, x, packed, qzeros, scales, y, k: int, n: int, workspace: torch.Tensor | None,
@@ -227,32 +223,24 @@ class W4A16Library:
         m = x.shape[0]
         ws_ptr = workspace.data_ptr() if workspace is not None else None
         ws_len = workspace.numel() * workspace.element_size() if workspace is not None else 0
-        with torch.cuda.device(x.device):
-            self.check(self.dll.w4a16_gemm_silu_mul(x.data_ptr(), packed.data_ptr(), qzeros.data_ptr(),
-                                                    scales.data_ptr(), y.data_ptr(), m, k, n, group_size, ws_ptr,
-                                                    ws_len, self._stream(x)),
-                       "w4a16_gemm_silu_mul")
+        self._launch(self.dll.w4a16_gemm_silu_mul, "w4a16_gemm_silu_mul", x, x.data_ptr(), packed.data_ptr(),
+                     qzeros.data_ptr(), scales.data_ptr(), y.data_ptr(), m, k, n, group_size, ws_ptr, ws_len)
         return y
 
     def add_rmsnorm(self, x, residual, weight, eps: float, x_norm, residual_out) -> torch.Tensor:
         """x_norm = RMSNorm(x + residual) * weight, residual_out = bf16(x + residual) (no add
         and no residual_out when residual is None); [M, K] bf16, contiguous, one GPU."""
         m, k = x.shape
-        with torch.cuda.device(x.device):
-            self.check(self.dll.w4a16_add_rmsnorm(x.data_ptr(), _ptr(residual), weight.data_ptr(), float(eps),
-                                                  x_norm.data_ptr(), _ptr(residual_out), m, k, self._stream(x)),
-                       "w4a16_add_rmsnorm")
+        self._launch(self.dll.w4a16_add_rmsnorm, "w4a16_add_rmsnorm", x, x.data_ptr(), _ptr(residual),
+                     weight.data_ptr(), float(eps), x_norm.data_ptr(), _ptr(residual_out), m, k)
         return x_norm
 
     def rmsnorm_strided(self, x, rows_inner: int, stride_outer: int, stride_inner: int, weight, eps: float,
                         x_norm, m: int, k: int) -> torch.Tensor:
         """x_norm [m, k] = RMSNorm of rows read at x + (r // rows_inner) * stride_outer +
         (r % rows_inner) * stride_inner (elements), no residual."""
-        with torch.cuda.device(x.device):
-            self.check(self.dll.w4a16_rmsnorm_strided(x.data_ptr(), rows_inner, stride_outer, stride_inner,
-                                                      weight.data_ptr(), float(eps), x_norm.data_ptr(), m, k,
-                                                      self._stream(x)),
-                       "w4a16_rmsnorm_strided")
+        self._launch(self.dll.w4a16_rmsnorm_strided, "w4a16_rmsnorm_strided", x, x.data_ptr(), rows_inner,
+                     stride_outer, stride_inner, weight.data_ptr(), float(eps), x_norm.data_ptr(), m, k)
         return x_norm
 
     def gemm_rmsnorm(self, x, residual, weight, eps: float, x_norm, residual_out, packed, qzeros, scales, y,
@@ -262,12 +250,10 @@ class W4A16Library:
         m, k = x.shape
         ws_ptr = workspace.data_ptr() if workspace is not None else None
         ws_len = workspace.numel() * workspace.element_size() if workspace is not None else 0
-        with torch.cuda.device(x.device):
-            self.check(self.dll.w4a16_gemm_rmsnorm(x.data_ptr(), _ptr(residual), weight.data_ptr(), float(eps),
-                                                   x_norm.data_ptr(), _ptr(residual_out), packed.data_ptr(),
-                                                   qzeros.data_ptr(), scales.data_ptr(), y.data_ptr(), m, k, n,
-                                                   group_size, int(silu_mul), ws_ptr, ws_len, self._stream(x)),
-                       "w4a16_gemm_rmsnorm")
+        self._launch(self.dll.w4a16_gemm_rmsnorm, "w4a16_gemm_rmsnorm", x, x.data_ptr(), _ptr(residual),
+                     weight.data_ptr(), float(eps), x_norm.data_ptr(), _ptr(residual_out), packed.data_ptr(),
+                     qzeros.data_ptr(), scales.data_ptr(), y.data_ptr(), m, k, n, group_size, int(silu_mul), ws_ptr,
+                     ws_len)
         return y
 
     def gemm_residual_stats(self, x, packed, qzeros, scales, residual, s_out, residual_out, ssq_out, k: int, n: int,
@@ -277,12 +263,9 @@ class W4A16Library:
         m = x.shape[0]
         ws_ptr = workspace.data_ptr() if workspace is not None else None
         ws_len = workspace.numel() * workspace.element_size() if workspace is not None else 0
-        with torch.cuda.device(x.device):
-            self.check(self.dll.w4a16_gemm_residual_stats(x.data_ptr(), packed.data_ptr(), qzeros.data_ptr(),
-                                                          scales.data_ptr(), residual.data_ptr(), s_out.data_ptr(),
-                                                          residual_out.data_ptr(), ssq_out.data_ptr(), m, k, n,
-                                                          group_size, ws_ptr, ws_len, self._stream(x)),
-                       "w4a16_gemm_residual_stats")
+        self._launch(self.dll.w4a16_gemm_residual_stats, "w4a16_gemm_residual_stats", x, x.data_ptr(),
+                     packed.data_ptr(), qzeros.data_ptr(), scales.data_ptr(), residual.data_ptr(), s_out.data_ptr(),
+                     residual_out.data_ptr(), ssq_out.data_ptr(), m, k, n, group_size, ws_ptr, ws_len)
 
     def gemm_rmsnorm_stats(self, s, ssq, weight, eps: float, x_norm, packed, qzeros, scales, y, n: int,
                            workspace: torch.Tensor | None, group_size: int = 128, silu_mul: bool = False):
@@ -290,12 +273,9 @@ class W4A16Library:
         m, k = s.shape
         ws_ptr = workspace.data_ptr() if workspace is not None else None
         ws_len = workspace.numel() * workspace.element_size() if workspace is not None else 0
-        with torch.cuda.device(s.device):
-            self.check(self.dll.w4a16_gemm_rmsnorm_stats(s.data_ptr(), ssq.data_ptr(), weight.data_ptr(), float(eps),
-                                                         _ptr(x_norm), packed.data_ptr(), qzeros.data_ptr(),
-                                                         scales.data_ptr(), y.data_ptr(), m, k, n, group_size,
-                                                         int(silu_mul), ws_ptr, ws_len, self._stream(s)),
-                       "w4a16_gemm_rmsnorm_stats")
+        self._launch(self.dll.w4a16_gemm_rmsnorm_stats, "w4a16_gemm_rmsnorm_stats", s, s.data_ptr(), ssq.data_ptr(),
+                     weight.data_ptr(), float(eps), _ptr(x_norm), packed.data_ptr(), qzeros.data_ptr(),
+                     scales.data_ptr(), y.data_ptr(), m, k, n, group_size, int(silu_mul), ws_ptr, ws_len)
         return y
 
     def gemm_config(self, x, packed, qzeros, scales, y, k: int, n: int, regime: int, p0: int, p1: int,
@@ -305,10 +285,9 @@ class W4A16Library:
         ws_ptr = workspace.data_ptr() if workspace is not None else None
         ws_len = workspace.numel() * workspace.element_size() if workspace is not None else 0
         fn = self.dll.w4a16_gemm_silu_mul_config if silu_mul else self.dll.w4a16_gemm_config
-        with torch.cuda.device(x.device):
-            self.check(fn(x.data_ptr(), packed.data_ptr(), qzeros.data_ptr(), scales.data_ptr(), y.data_ptr(), m, k,
-                          n, group_size, regime, p0, p1, p2, split, ws_ptr, ws_len, self._stream(x)),
-                       "w4a16_gemm_silu_mul_config" if silu_mul else "w4a16_gemm_config")
+        self._launch(fn, "w4a16_gemm_silu_mul_config" if silu_mul else "w4a16_gemm_config", x, x.data_ptr(),
+                     packed.data_ptr(), qzeros.data_ptr(), scales.data_ptr(), y.data_ptr(), m, k, n, group_size,
+                     regime, p0, p1, p2, split, ws_ptr, ws_len)
         return y
 
 

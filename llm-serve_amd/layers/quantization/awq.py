@@ -330,8 +330,8 @@ def _aligned16(t: torch.Tensor) -> bool:
     return t.data_ptr() % 16 == 0
 
 
-def _prepare_linear(inputs, packed_qweight, qzeros, scales, group_size):
-    """Shared argument checks of the GEMM entry points; returns (x [M, K], lead dims, K, N)."""
+def _check_linear(inputs, packed_qweight, qzeros, scales, group_size) -> None:
+    """The argument errors of the GEMM entry points, in the reference's order and words."""
     if not inputs.is_floating_point():
         raise ValueError("AWQ activations must use a floating dtype")
     if inputs.dtype != scales.dtype:
@@ -354,13 +354,39 @@ def _prepare_linear(inputs, packed_qweight, qzeros, scales, group_size):
         raise ValueError("packed qweight does not match the scales shape")
     if n % 64:
         raise ValueError("AWQ HIP GEMM requires the output size to be divisible by 64")
-    lead = inputs.shape[:-1]
-    x = inputs.reshape(-1, k)
+
+
+def _prepare_linear(inputs, packed_qweight, qzeros, scales, group_size):
+    """Shared argument checks of the GEMM entry points; returns (x [M, K], lead dims, K, N).
+    One expression accepts what every check of ``_check_linear`` accepts, and only what it
+    does not accept goes through them: they are most of the host time of a small call."""
+    bf16, i32 = torch.bfloat16, torch.int32
+    device = inputs.get_device()
+    if (inputs.dtype is bf16 and scales.dtype is bf16 and device >= 0 and group_size == 128
+            and packed_qweight.get_device() == device and qzeros.get_device() == device
+            and scales.get_device() == device and qzeros.dtype is i32 and packed_qweight.dtype is i32):
+        groups, n = scales.shape
+        k = groups * 128
+        shape = inputs.shape
+        if shape[-1] != k or packed_qweight.numel() * 8 != k * n or n % 64:
+            _check_linear(inputs, packed_qweight, qzeros, scales, group_size)
+    else:
+        _check_linear(inputs, packed_qweight, qzeros, scales, group_size)
+        n = scales.shape[1]
+        k = scales.shape[0] * group_size
+        shape = inputs.shape
+    x = inputs if len(shape) == 2 else inputs.reshape(-1, k)
     if not x.is_contiguous() or not _aligned16(x):
         x = x.contiguous()
         if not _aligned16(x):
             x = x.clone()
-    return x, lead, k, n
+    return x, shape[:-1], k, n
+
+
+@functools.lru_cache(maxsize=4096)
+def _workspace_bytes(m: int, k: int, n: int, group_size: int) -> int:
+    """The library's answer for these sizes, which depends on nothing else."""
+    return lib().workspace_bytes(m, k, n, group_size)
 
 
 def awq_linear(inputs: torch.Tensor, packed_qweight: torch.Tensor, qzeros: torch.Tensor, scales: torch.Tensor,
@@ -373,14 +399,14 @@ def awq_linear(inputs: torch.Tensor, packed_qweight: torch.Tensor, qzeros: torch
     per-device shared one."""
     x, lead, k, n = _prepare_linear(inputs, packed_qweight, qzeros, scales, group_size)
     m = x.shape[0]
-    y = torch.empty((m, n), dtype=inputs.dtype, device=inputs.device)
+    y = x.new_empty((m, n))
     if m == 0:
         return y.reshape(*lead, n)
     library = lib()
     if workspace is None:
-        workspace = WORKSPACE.get(inputs.device, library.workspace_bytes(m, k, n, group_size))
+        workspace = WORKSPACE.get(inputs.device, _workspace_bytes(m, k, n, group_size))
     library.gemm(x, packed_qweight, qzeros, scales.contiguous(), y, k, n, workspace, group_size)
-    return y.reshape(*lead, n)
+    return y if len(lead) == 1 else y.reshape(*lead, n)
 
 
 def awq_linear_residual(inputs: torch.Tensor, packed_qweight: torch.Tensor, qzeros: torch.Tensor,
@@ -407,7 +433,7 @@ def awq_linear_residual(inputs: torch.Tensor, packed_qweight: torch.Tensor, qzer
         return out
     library = lib()
     if workspace is None:
-        workspace = WORKSPACE.get(inputs.device, library.workspace_bytes(m, k, n, group_size))
+        workspace = WORKSPACE.get(inputs.device, _workspace_bytes(m, k, n, group_size))
     library.gemm_residual(x, packed_qweight, qzeros, scales.contiguous(), res, out.reshape(m, n), k, n, workspace,
                           group_size)
     return out
@@ -426,14 +452,14 @@ def awq_linear_silu_mul(inputs: torch.Tensor, packed_qweight: torch.Tensor, qzer
     if n % 128:
         raise ValueError("AWQ fused SiLU * up requires the gate|up output size to be divisible by 128")
     m = x.shape[0]
-    y = torch.empty((m, n // 2), dtype=inputs.dtype, device=inputs.device)
+    y = x.new_empty((m, n // 2))
     if m == 0:
         return y.reshape(*lead, n // 2)
     library = lib()
     if workspace is None:
-        workspace = WORKSPACE.get(inputs.device, library.workspace_bytes(m, k, n, group_size))
+        workspace = WORKSPACE.get(inputs.device, _workspace_bytes(m, k, n, group_size))
     library.gemm_silu_mul(x, packed_qweight, qzeros, scales.contiguous(), y, k, n, workspace, group_size)
-    return y.reshape(*lead, n // 2)
+    return y if len(lead) == 1 else y.reshape(*lead, n // 2)
 
 
 def _norm_operands(x: torch.Tensor, residual: torch.Tensor | None, weight: torch.Tensor, strided_ok: bool = False):
@@ -547,7 +573,7 @@ def awq_linear_rmsnorm(inputs: torch.Tensor, residual: torch.Tensor | None, norm
     if m > 0:
         library = lib()
         if workspace is None:
-            workspace = WORKSPACE.get(inputs.device, library.workspace_bytes(m, k, n, group_size))
+            workspace = WORKSPACE.get(inputs.device, _workspace_bytes(m, k, n, group_size))
         x_norm = torch.empty((m, k), dtype=torch.bfloat16, device=inputs.device)
         library.gemm_rmsnorm(xv, rv, norm_weight, eps, x_norm,
                              residual_out.view(m, k) if residual_out is not None else None, packed_qweight,
@@ -597,7 +623,7 @@ def awq_linear_residual_stats(inputs: torch.Tensor, packed_qweight: torch.Tensor
     if m > 0:
         library = lib()
         if workspace is None:
-            workspace = WORKSPACE.get(inputs.device, library.workspace_bytes(m, k, n, group_size))
+            workspace = WORKSPACE.get(inputs.device, _workspace_bytes(m, k, n, group_size))
         library.gemm_residual_stats(x, packed_qweight, qzeros, scales.contiguous(), res, s_out,
                                     residual_out.reshape(m, n), ssq, k, n, workspace, group_size)
     return NormInput(s_out, ssq), residual_out
@@ -641,7 +667,7 @@ def awq_linear_rmsnorm_stats(inp: NormInput, norm_weight: torch.Tensor, eps: flo
     if m > 0:
         library = lib()
         if workspace is None:
-            workspace = WORKSPACE.get(s.device, library.workspace_bytes(m, k, n, group_size))
+            workspace = WORKSPACE.get(s.device, _workspace_bytes(m, k, n, group_size))
         library.gemm_rmsnorm_stats(s, ssq, norm_weight, eps, x_norm, packed_qweight, qzeros, scales.contiguous(), y, n,
                                    workspace, group_size, silu_mul)
     return y

@@ -313,3 +313,21 @@ def test_runtime_config_reserves_for_the_engine_batch(awq):
     cfg = awq.AWQRuntimeConfig(bits=4, group_size=128, zero_point=True, version="gemm", backend="autoawq",
                                activation_dtype=torch.bfloat16)
     assert cfg.max_batched_tokens == 16384  # the reference engine's max_num_batched_tokens (config.py:11)
+
+
+def test_library_methods_refuse_host_tensors():
+    """The thin wrappers pass raw pointers on: a host tensor raises before any launch, with or
+    without a GPU in the machine."""
+    lib = importlib.import_module("llm-serve_amd").lib()
+    x = torch.zeros(1, 128, dtype=torch.bfloat16)
+    y = torch.zeros(1, 64, dtype=torch.bfloat16)
+    packed = torch.zeros(128 * 64 // 8, dtype=torch.int32)
+    qzeros = torch.zeros(1, 8, dtype=torch.int32)
+    scales = torch.zeros(1, 64, dtype=torch.bfloat16)
+    weight = torch.zeros(128, dtype=torch.bfloat16)
+    with pytest.raises(ValueError):
+        lib.gemm(x, packed, qzeros, scales, y, 128, 64, None)
+    with pytest.raises(ValueError):
+        lib.add_rmsnorm(x, None, weight, 1e-6, torch.empty_like(x), None)
+    with pytest.raises(ValueError):
+        lib.gemm_config(x, packed, qzeros, scales, y, 128, 64, 1, 1, 4, 1, None, p2=1)
