@@ -315,6 +315,29 @@ __device__ __forceinline__ void mma_group(WaveTile<WM, TW, false>& wt, const uin
 #pragma unroll
     for (int mt = 0; mt < WM; ++mt) a[mt] = *reinterpret_cast<const bf16x8_t*>(base + mt * 16 * kARowBytes);
   };
+  // The main MFMAs of a step, half the row blocks at a time, the column blocks within a half
+  // outermost and back and forth: neighbours in the issue order share an operand, three times
+  // in four (128-row tiles) the weights'.  The large tiles run at the power limit, where fewer
+  // operand changes are a higher clock; a register-only loop runs 0.8 % faster with the weights
+  // held than with the activations held.  Row blocks outermost over all rows before;
+  // MI355X, us (two layers in a graph; norm + gate_up + down): M = 200 292.4 -> 289.7,
+  // M = 320 355.0 -> 349.0, M = 497 148.2 -> 145.9, M = 2048 510.3 -> 504.6 (QKV alone with its
+  // norm, M = 1331: 73.6 -> 71.5).  All rows inside each column block spills in the 128 x 64
+  // wave tile (M = 2048: +6 %) and gains the same elsewhere; pairs of rows gain a third less.
+  auto main_mfmas = [&](const bf16x8_t (&a)[WM], const bf16x8_t (&bf)[TW]) {
+    constexpr int H = WM / 2;
+    static_assert(WM % 2 == 0, "two halves");
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int t = 0; t < TW; ++t)
+#pragma unroll
+        for (int m = 0; m < H; ++m) {
+          const int tt = h ? TW - 1 - t : t;
+          const int mt = h * H + (t & 1 ? H - 1 - m : m);
+          acc[mt][tt] = mfma16(a[mt], bf[tt], acc[mt][tt]);
+        }
+  };
   // A step's dequant issues every tile's scaling MFMAs before the first rounding reads one
   // (tile by tile, each rounding waits on the MFMA just issued: 0.3-2.3 % slower at M >= 128).
   auto dequant = [&](bf16x8_t (&bf)[TW], int j) {
@@ -327,7 +350,7 @@ __device__ __forceinline__ void mma_group(WaveTile<WM, TW, false>& wt, const uin
   if constexpr (WM * TW > 16) {
     // Large wave tiles: no register double-buffering (the 128 x 64 tile's accumulators
     // take half of the 256 registers a wave has at two waves per SIMD, and the kernel uses
-    // 250 of them); the WM x TW independent MFMAs of a step leave the scheduler enough
+    // them all); the WM x TW independent MFMAs of a step leave the scheduler enough
     // work to overlap.
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -335,10 +358,7 @@ __device__ __forceinline__ void mma_group(WaveTile<WM, TW, false>& wt, const uin
       bf16x8_t bf[TW];
       read_a(a, j);
       dequant(bf, j);
-#pragma unroll
-      for (int mt = 0; mt < WM; ++mt)
-#pragma unroll
-        for (int tt = 0; tt < TW; ++tt) acc[mt][tt] = mfma16(a[mt], bf[tt], acc[mt][tt]);
+      main_mfmas(a, bf);
     }
     return;
   }
@@ -363,10 +383,7 @@ __device__ __forceinline__ void mma_group(WaveTile<WM, TW, false>& wt, const uin
 #pragma unroll
         for (int tt = 0; tt < TW; ++tt) sd[tt] = dequant_scale(b.w[tt][j + 1], ts[tt], nib);
       }
-#pragma unroll
-      for (int mt = 0; mt < WM; ++mt)
-#pragma unroll
-        for (int tt = 0; tt < TW; ++tt) acc[mt][tt] = mfma16(a[c][mt], bf[c][tt], acc[mt][tt]);
+      main_mfmas(a[c], bf[c]);
       __builtin_amdgcn_sched_barrier(0);
       if (j < 3) {
 #pragma unroll
@@ -378,10 +395,7 @@ __device__ __forceinline__ void mma_group(WaveTile<WM, TW, false>& wt, const uin
       read_a(a[c ^ 1], j + 1);
       dequant(bf[c ^ 1], j + 1);
     }
-#pragma unroll
-    for (int mt = 0; mt < WM; ++mt)
-#pragma unroll
-      for (int tt = 0; tt < TW; ++tt) acc[mt][tt] = mfma16(a[c][mt], bf[c][tt], acc[mt][tt]);
+    main_mfmas(a[c], bf[c]);
   }
 }
 
