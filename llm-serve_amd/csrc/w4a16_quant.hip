@@ -153,6 +153,56 @@ __global__ __launch_bounds__(kQuantThreads) void quantize_kernel(const void* __r
 constexpr int kFastRows = 128;
 constexpr int kFastThreads = 4 * kFastRows;
 
+// Which blocks an XCD takes.  A block reads 256 bytes (bf16, groups of 128) of each of its rows
+// and writes 64 bytes of each input row's words, half a cache line; dispatched in grid order,
+// round-robin over the XCDs, no L2 holds both halves of a written line or neighbouring pieces
+// of a read row.  A weight that does not fit the 256 MB memory-side cache beside its output
+// goes in strips: each XCD takes a contiguous eighth of the blocks, in strips of kStrip row
+// blocks that walk the groups.  us a call, grid order against strips: 24576 x 4096 bf16 groups
+// of 128 / 64 61.0 -> 51.5 / 69.4 -> 54.5, 34816 x 5120 bf16 95.0 -> 91.3, 24576 x 4096 fp32
+// 94.9 -> 91.5, 4096 x 12288 fp32 50.8 -> 49.9.  (Strips of 1, 2, 8 and all row blocks: 1 - 5 %
+// slower than 4; non-temporal loads or stores 26 and 4 %.)  Smaller weights gain nothing (bf16
+// 19456 x 2560 28.1 / 28.0, 7168 x 5120 17.3 / 17.5), groups of 32 now and then (73.6 / 69.3 at
+// 24576 x 4096, 117.1 / 120.1 at 34816 x 5120): they keep the grid order.
+constexpr size_t kStripBytes = size_t{128} << 20;
+constexpr int kStrip = 4;
+
+struct QuantGrid {
+  int strips;                           // else grid order
+  int row_blocks, groups;
+  int per, rem;                         // the blocks of an XCD: per, the first rem XCDs one more
+  uint32_t strip_mul, strip_shift;      // n / (kStrip groups) = n strip_mul >> strip_shift, n < 2^31
+};
+
+static QuantGrid quant_grid(bool strips, int row_blocks, int groups) {
+  const uint32_t d = static_cast<uint32_t>(kStrip) * groups;
+  uint32_t shift = 31;
+  while ((1ull << (shift - 31)) < d) ++shift;
+  const int total = row_blocks * groups;
+  return QuantGrid{strips, row_blocks, groups, total >> 3, total & 7,
+                   static_cast<uint32_t>(((1ull << shift) + d - 1) / d), shift};
+}
+
+// No division: the index arithmetic runs ahead of the first load, and three divisions there
+// took 4 us of the 55.4 that the call then took.
+__device__ __forceinline__ void quant_block(const QuantGrid& q, int& row_block, int& group) {
+  if (!q.strips) {
+    row_block = blockIdx.x;
+    group = blockIdx.y;
+    return;
+  }
+  const int b = blockIdx.y * q.row_blocks + blockIdx.x;
+  const int xcd = b & 7;
+  const uint32_t n = xcd * q.per + (xcd < q.rem ? xcd : q.rem) + (b >> 3);
+  const int strip = static_cast<int>((static_cast<uint64_t>(n) * q.strip_mul) >> q.strip_shift);
+  const uint32_t at = n - strip * kStrip * q.groups;
+  const int width = q.row_blocks - strip * kStrip;  // row blocks of the last strip
+  if (width >= kStrip) group = at / kStrip;
+  else if (width == 3) group = at / 3;
+  else group = at / (width == 2 ? 2 : 1);
+  row_block = strip * kStrip + at - group * (width < kStrip ? width : kStrip);
+}
+
 // Smaller / larger of two, NaN if either is (torch's amin / amax), one instruction each.
 __device__ __forceinline__ float min_nan(float a, float b) { return __builtin_elementwise_minimum(a, b); }
 __device__ __forceinline__ float max_nan(float a, float b) { return __builtin_elementwise_maximum(a, b); }
@@ -168,15 +218,17 @@ template <int GS, int DTYPE>
 __global__ __launch_bounds__(kFastThreads) void quantize_rows_kernel(const void* __restrict__ weight,
                                                                      uint32_t* __restrict__ qweight,
                                                                      uint32_t* __restrict__ qzeros,
-                                                                     void* __restrict__ scales, int out_f, int in_f) {
+                                                                     void* __restrict__ scales, int out_f, int in_f,
+                                                                     QuantGrid grid) {
   constexpr int PART = GS / 4;       // values per thread
   constexpr int QP = GS + 4;         // LDS row pitch of the codes, bytes
   constexpr int PER = DTYPE == kDtypeF32 ? 4 : 8;  // values per 16-byte load
   static_assert(PART % PER == 0 && PART % 8 == 0, "a thread's values must split into 16-byte loads");
   __shared__ __attribute__((aligned(16))) uint8_t codes[kFastRows * QP];
   __shared__ float row_z[kFastRows];
-  const int o0 = blockIdx.x * kFastRows;
-  const int g = blockIdx.y;
+  int row_block, g;
+  quant_block(grid, row_block, g);
+  const int o0 = row_block * kFastRows;
   const int rows = out_f - o0 < kFastRows ? out_f - o0 : kFastRows;  // a multiple of 8
   const int tid = threadIdx.x;
   const int r = tid >> 2;  // the four threads of row r are adjacent lanes of one wave
@@ -314,16 +366,21 @@ size_t quantize_lds_bytes(int group_size) {
 template <int GS>
 static hipError_t launch_quantize_rows(const void* weight, int dtype, uint32_t* qweight, uint32_t* qzeros,
                                        void* scales, int out_f, int in_f, hipStream_t stream) {
-  const dim3 grid((out_f + kFastRows - 1) / kFastRows, in_f / GS);
+  const size_t bytes = static_cast<size_t>(out_f) * in_f * (dtype == kDtypeF32 ? 4 : 2);
+  const QuantGrid grid = quant_grid(GS >= 64 && bytes >= kStripBytes, (out_f + kFastRows - 1) / kFastRows, in_f / GS);
+  const dim3 blocks(grid.row_blocks, grid.groups);
   switch (dtype) {
     case kDtypeF32:
-      quantize_rows_kernel<GS, kDtypeF32><<<grid, kFastThreads, 0, stream>>>(weight, qweight, qzeros, scales, out_f, in_f);
+      quantize_rows_kernel<GS, kDtypeF32><<<blocks, kFastThreads, 0, stream>>>(weight, qweight, qzeros, scales, out_f,
+                                                                                  in_f, grid);
       break;
     case kDtypeF16:
-      quantize_rows_kernel<GS, kDtypeF16><<<grid, kFastThreads, 0, stream>>>(weight, qweight, qzeros, scales, out_f, in_f);
+      quantize_rows_kernel<GS, kDtypeF16><<<blocks, kFastThreads, 0, stream>>>(weight, qweight, qzeros, scales, out_f,
+                                                                                  in_f, grid);
       break;
     default:
-      quantize_rows_kernel<GS, kDtypeBF16><<<grid, kFastThreads, 0, stream>>>(weight, qweight, qzeros, scales, out_f, in_f);
+      quantize_rows_kernel<GS, kDtypeBF16><<<blocks, kFastThreads, 0, stream>>>(weight, qweight, qzeros, scales, out_f,
+                                                                                  in_f, grid);
   }
   return hipGetLastError();
 }
