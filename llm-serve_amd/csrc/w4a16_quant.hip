@@ -207,11 +207,12 @@ __device__ __forceinline__ void quant_block(const QuantGrid& q, int& row_block, 
 __device__ __forceinline__ float min_nan(float a, float b) { return __builtin_elementwise_minimum(a, b); }
 __device__ __forceinline__ float max_nan(float a, float b) { return __builtin_elementwise_maximum(a, b); }
 
-// clamp(n + z, 0, 15) as byte `e` of `word` (n, z whole numbers; the conversion clamps below
-// at 0 and takes NaN to 0).
+// clamp(n + z, 0, 15) as byte `E` of `word` (n, z whole numbers).  The conversion clamps below
+// at 0 and takes NaN to 0, so the minimum has to keep NaN: the quotients of a group with a NaN
+// or an infinity are code 0 here as in quantize_kernel.
 template <int E>
 __device__ __forceinline__ uint32_t put_code(uint32_t word, float n, float z) {
-  return __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fminf(n + z, 15.f), E, word);
+  return __builtin_amdgcn_cvt_pk_u8_f32(min_nan(n + z, 15.f), E, word);
 }
 
 template <int GS, int DTYPE>

@@ -192,3 +192,35 @@ def test_block_order_of_large_weights(cal, out_f, groups):
     parts = [cal.quantize_awq_weight(p.contiguous(), group_size=gs) for p in (w[:, :half], w[:, half:])]
     for name in ("qweight", "qzeros", "scales"):
         assert torch.equal(getattr(whole, name), torch.cat([getattr(p, name) for p in parts])), name
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("gs", [32, 64, 128])
+def test_non_finite_groups_as_the_general_kernel(cal, dtype, gs):
+    """Groups with a NaN, a +inf, a -inf, both, or nothing but NaN, beside finite groups of the
+    same rows: a weight that starts off a 16-byte boundary takes the general kernel, and both
+    give the same codes, zeros and scales (an undefined quotient is code 0)."""
+    rows, groups = 136, 3
+    w = (torch.randn((rows, groups, gs), generator=torch.Generator().manual_seed(gs)) * 0.05).to(dtype)
+    nan, inf = float("nan"), float("inf")
+    w[0, 0, 5] = nan
+    w[1, 0, gs - 1] = inf
+    w[2, 0, 0] = -inf
+    w[3, 0, 1], w[3, 0, 2] = inf, -inf
+    w[4, 0] = nan
+    w[5, 0] = inf
+    w[6, 0, 3], w[6, 0, 4] = inf, nan
+    w[130, 2, 7] = nan
+    w[135, 1, gs // 2] = -inf
+    w = w.view(rows, groups * gs).cuda()
+    store = torch.empty(w.numel() + 1, dtype=dtype, device="cuda")
+    off = store[1:].view_as(w).copy_(w)
+    assert w.data_ptr() % 16 == 0 and off.data_ptr() % 16 != 0
+    print(f"quantize non-finite {dtype} g{gs}", flush=True)
+    fast, general = cal.quantize_awq_weight(w, group_size=gs), cal.quantize_awq_weight(off, group_size=gs)
+    assert torch.equal(fast.qweight, general.qweight)
+    assert torch.equal(fast.qzeros, general.qzeros)
+    assert torch.equal(fast.scales.isnan(), general.scales.isnan())
+    assert torch.equal(fast.scales.nan_to_num(), general.scales.nan_to_num())
+    codes = ora.unpack_awq_int4(fast.qweight.cpu().numpy())[:gs]  # the first group, [position, row]
+    assert not codes[:, [0, 3, 4, 6]].any() and codes[gs - 1, 1] == 0
