@@ -365,8 +365,7 @@ def _prepare_linear(inputs, packed_qweight, qzeros, scales, group_size):
     if (inputs.dtype is bf16 and scales.dtype is bf16 and device >= 0 and group_size == 128
             and packed_qweight.get_device() == device and qzeros.get_device() == device
             and scales.get_device() == device and qzeros.dtype is i32 and packed_qweight.dtype is i32):
-        groups, n = scales.shape
-        k = groups * 128
+        k, n = scales.shape[0] * 128, scales.shape[1]
         shape = inputs.shape
         if shape[-1] != k or packed_qweight.numel() * 8 != k * n or n % 64:
             _check_linear(inputs, packed_qweight, qzeros, scales, group_size)

@@ -352,6 +352,18 @@ def test_leading_dims_are_flattened(gpu_lib):
     assert_gemm_close(y.reshape(6, n), full_reference(x.reshape(6, k), qw, qz, s))
 
 
+def test_scales_with_a_trailing_dimension_of_one(gpu_lib):
+    """scales [K/128, N, 1] is accepted as [K/128, N]: only the first two sizes are looked at."""
+    k, n = 256, 128
+    qw, qz, s = random_awq_gpu(k, n, seed=13)
+    awq = awq_mod()
+    packed = awq.repack_awq_qweight(qw)
+    x = random_x_gpu(3, k, seed=2)
+    for fn in (awq.awq_linear, awq.awq_linear_silu_mul):
+        want = fn(x, packed, qz, s, group_size=128)
+        assert torch.equal(fn(x, packed, qz, s.unsqueeze(-1), group_size=128), want)
+
+
 def test_too_small_workspace_is_an_error(gpu_lib):
     k, n, m = 12288, 4096, 16  # the down projection: split-K, so a workspace is needed
     qw, qz, s = random_awq_gpu(k, n, seed=5)
