@@ -382,6 +382,12 @@ def _prepare_linear(inputs, packed_qweight, qzeros, scales, group_size):
     return x, shape[:-1], k, n
 
 
+def _new_output(x: torch.Tensor, m: int, n: int) -> torch.Tensor:
+    """A bf16 [m, n] on x's GPU, a plain tensor whatever x's class.  (empty_strided parses its
+    arguments faster than empty; x.new_empty would hand on the class.)"""
+    return torch.empty_strided((m, n), (n, 1), dtype=torch.bfloat16, device=x.device)
+
+
 @functools.lru_cache(maxsize=4096)
 def _workspace_bytes(m: int, k: int, n: int, group_size: int) -> int:
     """The library's answer for these sizes, which depends on nothing else."""
@@ -398,7 +404,7 @@ def awq_linear(inputs: torch.Tensor, packed_qweight: torch.Tensor, qzeros: torch
     per-device shared one."""
     x, lead, k, n = _prepare_linear(inputs, packed_qweight, qzeros, scales, group_size)
     m = x.shape[0]
-    y = x.new_empty((m, n))
+    y = _new_output(x, m, n)
     if m == 0:
         return y.reshape(*lead, n)
     library = lib()
@@ -451,7 +457,7 @@ def awq_linear_silu_mul(inputs: torch.Tensor, packed_qweight: torch.Tensor, qzer
     if n % 128:
         raise ValueError("AWQ fused SiLU * up requires the gate|up output size to be divisible by 128")
     m = x.shape[0]
-    y = x.new_empty((m, n // 2))
+    y = _new_output(x, m, n // 2)
     if m == 0:
         return y.reshape(*lead, n // 2)
     library = lib()

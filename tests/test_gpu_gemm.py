@@ -364,6 +364,24 @@ def test_scales_with_a_trailing_dimension_of_one(gpu_lib):
         assert torch.equal(fn(x, packed, qz, s.unsqueeze(-1), group_size=128), want)
 
 
+def test_outputs_are_plain_tensors(gpu_lib):
+    """Activations of a torch.Tensor subclass give plain tensors, in every leading shape."""
+
+    class Activations(torch.Tensor):
+        pass
+
+    k, n = 256, 128
+    qw, qz, s = random_awq_gpu(k, n, seed=14)
+    awq = awq_mod()
+    packed = awq.repack_awq_qweight(qw)
+    for shape in ((k,), (3, k), (1, 2, k), (0, k)):
+        x = random_x_gpu(int(np.prod(shape[:-1])), k, seed=3).reshape(shape)
+        for fn in (awq.awq_linear, awq.awq_linear_silu_mul):
+            want = fn(x, packed, qz, s, group_size=128)
+            got = fn(x.as_subclass(Activations), packed, qz, s, group_size=128)
+            assert type(got) is torch.Tensor and torch.equal(got, want), (shape, fn.__name__)
+
+
 def test_too_small_workspace_is_an_error(gpu_lib):
     k, n, m = 12288, 4096, 16  # the down projection: split-K, so a workspace is needed
     qw, qz, s = random_awq_gpu(k, n, seed=5)
