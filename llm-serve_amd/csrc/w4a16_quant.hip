@@ -153,18 +153,36 @@ __global__ __launch_bounds__(kQuantThreads) void quantize_kernel(const void* __r
 constexpr int kFastRows = 128;
 constexpr int kFastThreads = 4 * kFastRows;
 
-// Which blocks an XCD takes.  A block reads 256 bytes (bf16, groups of 128) of each of its rows
-// and writes 64 bytes of each input row's words, half a cache line; dispatched in grid order,
-// round-robin over the XCDs, no L2 holds both halves of a written line or neighbouring pieces
-// of a read row.  A weight that does not fit the 256 MB memory-side cache beside its output
-// goes in strips: each XCD takes a contiguous eighth of the blocks, in strips of kStrip row
-// blocks that walk the groups.  us a call, grid order against strips: 24576 x 4096 bf16 groups
-// of 128 / 64 61.0 -> 51.5 / 69.4 -> 54.5, 34816 x 5120 bf16 95.0 -> 91.3, 24576 x 4096 fp32
-// 94.9 -> 91.5, 4096 x 12288 fp32 50.8 -> 49.9.  (Strips of 1, 2, 8 and all row blocks: 1 - 5 %
-// slower than 4; non-temporal loads or stores 26 and 4 %.)  Smaller weights gain nothing (bf16
-// 19456 x 2560 28.1 / 28.0, 7168 x 5120 17.3 / 17.5), groups of 32 now and then (73.6 / 69.3 at
-// 24576 x 4096, 117.1 / 120.1 at 34816 x 5120): they keep the grid order.
-constexpr size_t kStripBytes = size_t{128} << 20;
+// Which blocks an XCD takes: all in grid order, round-robin, or in strips -- each XCD a
+// contiguous eighth of the blocks, in strips of kStrip row blocks that walk the groups.
+//
+// A block reads 256 bytes (bf16, groups of 128) of each of its rows and writes 64 bytes, half a
+// cache line, of each input row's words.  In grid order the blocks in flight read one group's
+// column of the weight, pieces a row pitch apart, and no L2 holds both halves of a written line.
+// What decides is the pitch: 22016 rows of 4096 bf16 take 57.7 us in grid order and 49.5 in
+// strips, the same rows of 4224 (3 % more data) 50.9 in either, as if the pieces a multiple of
+// 4 KiB apart fell on few memory channels.  Measured over 70 shapes, grid order ->
+// strips in us a call, groups of 128 / 64:
+//   4 KiB pitch   64 MiB   8192 x 4096 bf16     21.3 -> 21.6 / 21.1 -> 21.2
+//                 80 MiB   10240 x 4096 bf16    25.3 -> 24.7 / 25.7 -> 25.3
+//                 96 MiB   12288 x 4096 bf16    32.9 -> 29.2 / 33.0 -> 29.9
+//                192 MiB   24576 x 4096 bf16    64.5 -> 51.9 / 69.1 -> 54.8
+//                448 MiB   28672 x 8192 bf16   173.3 -> 119.7 / 199.9 -> 122.4
+//                340 MiB   17408 x 5120 fp32    97.7 -> 90.1 / 99.2 -> 83.8
+//   others       130 MiB   26624 x 2560 bf16    40.1 -> 38.8 / 39.8 -> 39.2
+//                170 MiB   17408 x 5120 bf16    48.9 -> 49.6 / 49.2 -> 49.7
+//                170 MiB   5120 x 17408 bf16    50.5 -> 52.2 / 49.3 -> 51.3
+//                172 MiB   8192 x 11008 bf16    58.3 -> 52.2 / 58.6 -> 53.1
+//                190 MiB   19456 x 2560 fp32    50.6 -> 52.4 / 47.4 -> 48.1
+//                340 MiB   34816 x 5120 bf16    95.9 -> 92.0 / 95.0 -> 94.9
+// With a pitch of 4 KiB multiples strips gain up to 39 % from 80 MiB on (at worst +4 %: 5120 x
+// 17408 fp32); with other pitches nothing below 128 MiB, and -10 to +4 % from there on, where the
+// gains outweigh the losses.  Hence the two sizes.  (24576 x 4096 bf16 in strips of 1, 2, 8 and
+// all row blocks: 1 - 5 % slower than 4; non-temporal loads or stores 26 and 4 %.)  Groups of 32
+// gain nothing at any size and keep the grid order.
+constexpr size_t kStripPitch = 4096;
+constexpr size_t kStripBytes = size_t{80} << 20;
+constexpr size_t kStripBytesOther = size_t{128} << 20;
 constexpr int kStrip = 4;
 
 struct QuantGrid {
@@ -367,8 +385,9 @@ size_t quantize_lds_bytes(int group_size) {
 template <int GS>
 static hipError_t launch_quantize_rows(const void* weight, int dtype, uint32_t* qweight, uint32_t* qzeros,
                                        void* scales, int out_f, int in_f, hipStream_t stream) {
-  const size_t bytes = static_cast<size_t>(out_f) * in_f * (dtype == kDtypeF32 ? 4 : 2);
-  const QuantGrid grid = quant_grid(GS >= 64 && bytes >= kStripBytes, (out_f + kFastRows - 1) / kFastRows, in_f / GS);
+  const size_t pitch = static_cast<size_t>(in_f) * (dtype == kDtypeF32 ? 4 : 2);
+  const bool strips = GS >= 64 && out_f * pitch >= (pitch % kStripPitch == 0 ? kStripBytes : kStripBytesOther);
+  const QuantGrid grid = quant_grid(strips, (out_f + kFastRows - 1) / kFastRows, in_f / GS);
   const dim3 blocks(grid.row_blocks, grid.groups);
   switch (dtype) {
     case kDtypeF32:

@@ -177,18 +177,24 @@ def test_quotients_near_half_and_row_block_edges(cal, dtype, gs):
         np.testing.assert_array_equal(scale_array(p.scales), sc)
 
 
-@pytest.mark.parametrize("out_f,groups", [(136, 7713), (264, 3973), (392, 2677), (520, 2019), (904, 1161), (131976, 9)])
+@pytest.mark.parametrize("out_f,groups", [(136, 7713), (264, 3973), (392, 2677), (520, 2019), (904, 1161), (131976, 9),
+                                          (136, 4832), (264, 2496), (392, 1696), (520, 1280), (904, 736)])
 def test_block_order_of_large_weights(cal, out_f, groups):
-    """From 128 MiB on, blocks are dealt to the XCDs in eighths, in strips of four row blocks: last
-    strips of one to four row blocks (the last of 8 rows), even and uneven eighths.  The two
-    halves of the same weight stay below that size and go in grid order."""
+    """From 128 MiB on (80 MiB where the row pitch is a multiple of 4 KiB: the second line of
+    shapes), blocks are dealt to the XCDs in eighths, in strips of four row blocks: last strips of
+    one to four row blocks (the last of 8 rows), even and uneven eighths.  The two halves of the
+    same weight stay below that size and go in grid order."""
     gs = 64
     gen = torch.Generator(device="cuda").manual_seed(out_f)
     w = torch.randn((out_f, gs * groups), generator=gen, device="cuda").to(torch.bfloat16)
-    assert w.numel() * 2 >= 128 << 20
+    half = gs * (groups // 2)
+
+    def strips(cols):
+        return out_f * cols * 2 >= (80 << 20 if cols * 2 % 4096 == 0 else 128 << 20)
+
+    assert strips(gs * groups) and not strips(half) and not strips(gs * groups - half)
     print(f"quantize strips rows={out_f} groups={groups}", flush=True)
     whole = cal.quantize_awq_weight(w, group_size=gs)
-    half = gs * (groups // 2)
     parts = [cal.quantize_awq_weight(p.contiguous(), group_size=gs) for p in (w[:, :half], w[:, half:])]
     for name in ("qweight", "qzeros", "scales"):
         assert torch.equal(getattr(whole, name), torch.cat([getattr(p, name) for p in parts])), name
