@@ -345,3 +345,48 @@ def test_workspace_reserved_at_load_and_never_grown_in_capture(gpu_lib, monkeypa
         assert awq.WORKSPACE.get(torch.device("cuda"), have) is not None  # within the reserve: no allocation
         with pytest.raises(RuntimeError, match="graph capture"):
             awq.WORKSPACE.get(torch.device("cuda"), have + 1)
+
+
+@pytest.mark.parametrize("k", [128, 1024])
+@pytest.mark.parametrize("magnitude,eps", [(1.0, 1e-6), (1.0, 0.37), (2.0 ** -66, 0.0), (2.0 ** 60, 0.0)])
+def test_row_scale_is_the_rounded_reciprocal_root(gpu_lib, k, magnitude, eps):
+    """The row scale is 1 / sqrt(v) of 64 bits rounded to fp32, not one ulp of that off.  A row's
+    first element alone makes v; the others are placed where the scale times them lies at the
+    midpoint of two bf16 values, so that a scale one ulp up or down rounds some of them
+    differently (in half of the rows at least: checked on the oracle)."""
+    m = 4096
+    rng = np.random.default_rng(k)
+    a = (magnitude * rng.integers(2048, 4096, m) / 2048).astype(np.float32)  # 12 bits: a * a is exact
+    v = (a * a / np.float32(k) + np.float32(eps)).astype(np.float32)  # the rest vanishes beside it
+
+    def scale(v):
+        return (1.0 / np.sqrt(v.astype(np.float64))).astype(np.float32)
+
+    r = scale(v)
+    j = np.arange(k - 1)
+    midpoints = 2.0 ** (np.floor(np.log2(magnitude * float(r[0]))) - 20 - j // 128) * (1 + (2 * (j % 128) + 1) / 256)
+    row = np.concatenate([a[:, None], midpoints / r.astype(np.float64)[:, None]], axis=1)
+    x_bits = ora.f32_to_bf16_bits(row.astype(np.float32))
+    r_bits = ora.f32_to_bf16_bits((row - ora.bf16_bits_to_f32(x_bits)).astype(np.float32))
+    s = ora.bf16_bits_to_f32(x_bits) + ora.bf16_bits_to_f32(r_bits)
+
+    def normed(rstd):
+        return ora.f32_to_bf16_bits(s * rstd[:, None])
+
+    want = normed(r)
+    for other in (np.nextafter(r, np.float32(np.inf)), np.nextafter(r, np.float32(0))):
+        assert (normed(other) != want).any(axis=1).mean() > 0.5
+    print(f"row scale k={k} magnitude={magnitude} eps={eps}", flush=True)
+    out, _ = awq_mod().add_rms_norm(bf16_from_bits(x_bits), bf16_from_bits(r_bits),
+                                    torch.ones(k, dtype=torch.bfloat16, device="cuda"), eps)
+    np.testing.assert_array_equal(bits_of(out), want)
+
+
+@pytest.mark.parametrize("k", [128, 1024])
+def test_row_scale_at_zero_and_infinity(gpu_lib, k):
+    """A zero row without eps (v = 0, an infinite scale: NaN as in the reference) and a row whose
+    sum of squares overflows (v = inf: zeros)."""
+    x = torch.zeros((2, k), dtype=torch.bfloat16, device="cuda")
+    x[1] = 3e38
+    out = awq_mod().add_rms_norm(x, None, torch.ones(k, dtype=torch.bfloat16, device="cuda"), 0.0)
+    assert bool(out[0].isnan().all()) and bool((out[1] == 0).all())
