@@ -141,12 +141,16 @@ template <bool RES, int C>
 hipError_t launch_whole(const uint16_t* x, const uint16_t* residual, const uint16_t* weight, uint16_t* x_norm,
                         uint16_t* residual_out, int M, int K, int rows_inner, int64_t stride_outer,
                         int64_t stride_inner, float eps, hipStream_t stream) {
-  if (rows_inner >= M && stride_inner == K)  // contiguous rows: no division ahead of the loads
-    add_rmsnorm_kernel<RES, C, false><<<M, kNormThreads, 0, stream>>>(x, residual, weight, x_norm, residual_out, K,
-                                                                     rows_inner, stride_outer, stride_inner, eps);
-  else
-    add_rmsnorm_kernel<RES, C, true><<<M, kNormThreads, 0, stream>>>(x, residual, weight, x_norm, residual_out, K,
-                                                                    rows_inner, stride_outer, stride_inner, eps);
+  if constexpr (!RES) {  // (rows with a residual are contiguous)
+    if (rows_inner < M || stride_inner != K) {
+      add_rmsnorm_kernel<RES, C, true><<<M, kNormThreads, 0, stream>>>(x, residual, weight, x_norm, residual_out, K,
+                                                                      rows_inner, stride_outer, stride_inner, eps);
+      return hipGetLastError();
+    }
+  }
+  // contiguous rows: no division ahead of the loads
+  add_rmsnorm_kernel<RES, C, false><<<M, kNormThreads, 0, stream>>>(x, residual, weight, x_norm, residual_out, K,
+                                                                   rows_inner, stride_outer, stride_inner, eps);
   return hipGetLastError();
 }
 
