@@ -65,8 +65,8 @@ __global__ __launch_bounds__(256) void dequant_awq_kernel(const uint32_t* __rest
 // per output word, gathering its two words from memory, read them in 8-byte pieces of rows
 // N / 2 bytes apart, four times over: 58 us for 4096 x 24576.)
 //
-// VEC: qweight and packed 16-byte aligned and rows a multiple of 16 bytes; otherwise one word
-// per load and store.
+// VEC: qweight 16-byte aligned and rows a multiple of 16 bytes; otherwise one word per load
+// (packed is 16-byte aligned, the API's own condition).
 constexpr int kRepackTiles = 16;
 constexpr int kRepackWords = 2 * kRepackTiles;   // AutoAWQ words per row of the block
 constexpr int kRepackPitch = kRepackWords + 4;   // LDS row pitch: 16-byte rows, 2-way conflicts at most
@@ -122,12 +122,7 @@ __global__ __launch_bounds__(256) void repack_kernel(const uint32_t* __restrict_
       }
       out[js] = w;
     }
-    if constexpr (VEC) {
-      *reinterpret_cast<uint4*>(dst + 4 * slot) = make_uint4(out[0], out[1], out[2], out[3]);
-    } else {
-#pragma unroll
-      for (int js = 0; js < 4; ++js) dst[4 * slot + js] = out[js];
-    }
+    *reinterpret_cast<uint4*>(dst + 4 * slot) = make_uint4(out[0], out[1], out[2], out[3]);
   }
 }
 
@@ -181,8 +176,7 @@ hipError_t launch_dequant(const uint32_t* qweight, const uint32_t* qzeros, const
 hipError_t launch_repack(const uint32_t* qweight, uint32_t* packed, int K, int N, hipStream_t stream) {
   const int blocks_n = (N / kTileCols + kRepackTiles - 1) / kRepackTiles;
   const unsigned grid = static_cast<unsigned>(K / kGroup) * static_cast<unsigned>(blocks_n);
-  const bool vec = N % 32 == 0 && reinterpret_cast<uintptr_t>(qweight) % 16 == 0 &&
-                   reinterpret_cast<uintptr_t>(packed) % 16 == 0;
+  const bool vec = N % 32 == 0 && reinterpret_cast<uintptr_t>(qweight) % 16 == 0;
   if (vec) repack_kernel<true><<<grid, 256, 0, stream>>>(qweight, packed, N, blocks_n);
   else repack_kernel<false><<<grid, 256, 0, stream>>>(qweight, packed, N, blocks_n);
   return hipGetLastError();
