@@ -43,7 +43,8 @@ __device__ __forceinline__ TileCoord tile_coord(int b, int m_blocks, int n_block
 
 // A wave's output tile of TW 16-column layout tiles x 16 WM rows, on one of two matrix
 // instructions:
-//   WIDE   v_mfma_f32_32x32x16_bf16 over blocks of 32 rows x 32 columns (pairs of layout tiles);
+//   WIDE   v_mfma_f32_32x32x16_bf16 over blocks of 32 rows x 32 columns (TW = 2: one block of
+//          two layout tiles wide);
 //   else   v_mfma_f32_16x16x32_bf16 over blocks of 16 x 16.
 // A 32x32x16 does the work of two 16x16x32 in the same 32 cycles and takes the issue port
 // once.  Register-only loops with two waves on a SIMD and three VALU instructions per 16
@@ -60,7 +61,10 @@ __device__ __forceinline__ TileCoord tile_coord(int b, int m_blocks, int n_block
 // in any order that A follows: fragment 2 js + ab of 32-row step js takes rows {8 ab ..} and
 // {16 + 8 ab ..}, so lane l loads tile pair member (l / 16) % 2, lane slot (l % 16) +
 // 32 (l / 32) + 16 ab -- a permutation of the load addresses, no data movement -- and A reads
-// the same rows' chunks 4 js + 2 (l / 32) + ab.
+// the same rows' chunks 4 js + 2 (l / 32) + ab.  The products of an output are then summed in
+// another order than in the narrow form, both in fp32: at M = 129 and 192, K = 128 to 17408, up
+// to 5 in 10,000 bf16 outputs round the other way, and the error against 64 bits is the same to
+// six digits (1.66e-3, the rounding of the output).
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(3))) uint8_t lds_u8_t;
 typedef __attribute__((address_space(3))) void lds_void_t;
@@ -68,16 +72,13 @@ typedef __attribute__((address_space(3))) void lds_void_t;
 template <int WM, int TW, bool WIDE>
 struct WaveTile {
   static constexpr bool kWide = WIDE;
-  static_assert(!WIDE || TW % 2 == 0, "pairs of layout tiles");
+  static_assert(!WIDE || (TW == 2 && WM % 2 == 0), "one 32-column block of 32-row blocks");
   static constexpr int kTiles = TW;
   static constexpr int kSteps = kWide ? 8 : 4;      // matrix steps of a 128-deep group
   static constexpr int MT = kWide ? WM / 2 : WM;    // row blocks
   static constexpr int NT = kWide ? TW / 2 : TW;    // column blocks
   static constexpr int Q = kWide ? 4 : 1;           // 16-byte fragments per block
-  static constexpr int kRows = kWide ? 32 : 16;     // rows of a block
   static constexpr int kCols = kWide ? 32 : 16;     // columns of a block
-  static constexpr int kFrags = MT * NT * Q;        // WM TW 16-byte fragments per lane
-  static_assert(!kWide || WM % 2 == 0, "32-row blocks");
   typedef std::conditional_t<kWide, f32x16_t, f32x4_t> acc_t;
   acc_t acc[MT][NT];
 
@@ -135,7 +136,7 @@ struct BGroup {
   // Word of matrix step s in column block nt: the 4 words of a load are 32-row steps, and a
   // wide block has two loads, one per half of the rows.
   __device__ __forceinline__ uint32_t word(int nt, int s) const {
-    if constexpr (Wt::kWide) return w[2 * nt + s % 2][s / 2];
+    if constexpr (Wt::kWide) return w[s % 2][s / 2];
     else return w[nt][s];
   }
 };
@@ -154,6 +155,7 @@ struct BSources {
 template <class Wt, bool LOAD_SC>
 __device__ __forceinline__ void load_b_group(BGroup<Wt>& b, const BSources& src, int g, bool active, int N, int t0,
                                              int dt, int lane) {
+  static_assert(!Wt::kWide || !LOAD_SC, "the wide form's scales are staged");
   constexpr int TW = Wt::kTiles;
   const int NT16 = N / kTileCols;
   const int c = lane & 15;
@@ -165,8 +167,8 @@ __device__ __forceinline__ void load_b_group(BGroup<Wt>& b, const BSources& src,
     const int gw = static_cast<int>(static_cast<uint32_t>(g) * NT16 * 1024u);
     if constexpr (Wt::kWide) {
       const uint32_t wo = oob + static_cast<uint32_t>(t * 64 + (lane & 47)) * 16u;
-      b.w[2 * nt] = __builtin_amdgcn_raw_buffer_load_b128(src.w, wo, gw, 0);
-      b.w[2 * nt + 1] = __builtin_amdgcn_raw_buffer_load_b128(src.w, wo + 256u, gw, 0);
+      b.w[0] = __builtin_amdgcn_raw_buffer_load_b128(src.w, wo, gw, 0);
+      b.w[1] = __builtin_amdgcn_raw_buffer_load_b128(src.w, wo + 256u, gw, 0);
     } else {
       b.w[nt] = __builtin_amdgcn_raw_buffer_load_b128(src.w, oob | (static_cast<uint32_t>(t * 64 + lane) * 16u), gw, 0);
     }
@@ -549,7 +551,8 @@ __device__ __forceinline__ void finish_tile(WaveTile<WM, TW, WIDE>& wt, StageFn 
   }
 
   if (o.split > 1) {
-    // Every workgroup stores its fp32 fragments (lane-major, 1 KiB per 16 x 16 MFMA tile)
+    // Every workgroup stores its fp32 fragments (lane-major, 1 KiB each: a 16 x 16
+    // accumulator tile, or a quarter of a 32 x 32 one)
     // into partials[sidx][tile][wave of slice 0]; the last to arrive sums all splits in
     // split order, KC fragments at a time so that the loads of a chunk share one wait.  Only
     // slice 0 holds results; the other slices take part in the barriers alone.
@@ -711,7 +714,7 @@ __device__ __forceinline__ void finish_tile(WaveTile<WM, TW, WIDE>& wt, StageFn 
           }
       store_rows(std::integral_constant<int, CPR>{}, o.col_w + 16 * TP * part);
     }
-  } else if constexpr (Wt::kWide && TW == 2) {
+  } else if constexpr (Wt::kWide) {
     // One column block: gate columns in the lanes with lane / 16 even, their up columns 16
     // lanes on.  Half of each lane's values change places, so that every lane holds both
     // operands of half of the rows: gate lanes those of fragments 0 and 1, up lanes of 2, 3.
@@ -733,28 +736,27 @@ __device__ __forceinline__ void finish_tile(WaveTile<WM, TW, WIDE>& wt, StageFn 
         *reinterpret_cast<uint16_t*>(ep + off) = f32_to_bf16_bits(silu_mul_of_bf16(__uint_as_float(gu[0]), __uint_as_float(gu[1])));
       }
     store_rows(std::integral_constant<int, CPR>{}, o.col_w);
-  } else if constexpr (TW % 2 == 0) {  // the fused product pairs the two halves of a wave's blocks
-    constexpr int H = Wt::NT / 2;                // gate blocks
-    constexpr int HT = TW / 2;                   // gate tiles
-    constexpr int TP0 = HT % kParts == 0 && HT / kParts * 16 >= Wt::kCols ? HT / kParts : HT;
-    constexpr int TP = TP0 & -TP0;               // gate tiles per pass (a power of two)
-    constexpr int NB = 16 * TP / Wt::kCols;      // gate blocks per pass
+  } else if constexpr (TW % 2 == 0) {  // the fused product pairs the two halves of a wave's tiles
+    constexpr int H = TW / 2;
+    constexpr int TP0 = (H % kParts == 0) ? H / kParts : H;
+    constexpr int TP = TP0 & -TP0;  // gate tiles per pass (a power of two)
+    constexpr int NP = H / TP;
     constexpr int CPR = 2 * TP;
     constexpr int PITCH = 16 * CPR;
     static_assert(WR * PITCH <= kRegion, "a pass fits the wave's region");
 #pragma unroll
-    for (int part = 0; part < H / NB; ++part) {
+    for (int part = 0; part < NP; ++part) {
 #pragma unroll
-      for (int mt = 0; mt < Wt::MT; ++mt)
+      for (int mt = 0; mt < WM; ++mt)
 #pragma unroll
-        for (int nt = 0; nt < NB; ++nt)
+        for (int t = 0; t < TP; ++t)
 #pragma unroll
-          for (int e = 0; e < 4 * Wt::Q; ++e) {
-            const int r = Wt::row(mt, e / 4, e % 4, lane);
-            const int c = Wt::col(nt, lane);
+          for (int i = 0; i < 4; ++i) {
+            const int r = 16 * mt + 4 * (lane >> 4) + i;
+            const int c = 16 * t + (lane & 15);
             const int off = r * PITCH + (((c >> 3) ^ (r % CPR)) << 4) + ((c & 7) << 1);
-            const int g = part * NB + nt;
-            *reinterpret_cast<uint16_t*>(ep + off) = f32_to_bf16_bits(silu_mul_of_bf16(wt.acc[mt][g][e], wt.acc[mt][g + H][e]));
+            const int tt = part * TP + t;
+            *reinterpret_cast<uint16_t*>(ep + off) = f32_to_bf16_bits(silu_mul_of_bf16(wt.acc[mt][tt][i], wt.acc[mt][tt + H][i]));
           }
       store_rows(std::integral_constant<int, CPR>{}, o.col_w + 16 * TP * part);
     }
