@@ -211,6 +211,9 @@ GemmPlan plan_decode(int M, int K, int N) {
 // to M = 2048 (beyond M = 1024 for widths below 4096 only: wider layers fill rounds with the
 // rules' 384- and 512-column tiles, which the model leaves out -- Qwen3-4B QKV 2560 x 6144
 // at M = 2048: 58.8 us on 128 x 384 tiles against 69.6 us on the model's 64 x 96).
+// The 96 x 256 and 64 x 256 constants, here and in the candidate tables below, were measured on
+// tile_kernel; since those tiles run on roll_kernel they are 8 - 17 % faster alone (gate_up
+// M = 192 50.3 -> 45.9 us on 96 x 256) than these give.  Not refitted.
 struct ModelTile {
   int wm, shape, occ, bm, bn;
   double alpha, beta;

@@ -4,16 +4,19 @@
 // Workgroup = NWM x NWN waves, output tile BM x BN (BM = 16 WM NWM, BN = 16 TW NWN).  Wave
 // (wm, wn) owns TW 16-column layout tiles (columns [16 TW wn, 16 TW (wn + 1)) of the tile)
 // and rows [16 WM wm, 16 WM (wm + 1)): WM x TW accumulator tiles of
-// v_mfma_f32_16x16x32_bf16.  Each wave dequantizes its own columns on the matrix cores
-// straight from its 16-byte loads into MFMA B fragments -- bf16_rne((q - z) s), the
-// reference's weights, see dequant_step -- with no LDS round trip, so a weight is
-// dequantized NWM times per workgroup and used for 16 WM rows each time: the dequant work
-// per main MFMA falls as 1 / WM whatever TW is.  The activation tile (BM rows x one 128-deep
-// group) is shared by all waves through LDS: it is brought in by direct-to-LDS 16-byte
-// buffer loads, one or two groups per batch with the next batch in flight while one is
-// computed, in a row-major layout whose sixteen 16-byte chunks per row are XOR-swizzled by
-// (row & 15): the 16 lanes reading one fragment chunk (16 consecutive rows) then hit 16
-// different chunk positions, i.e. all 64 LDS banks once.  The scales and zero words of the
+// v_mfma_f32_16x16x32_bf16 in tile_kernel, WM / 2 x 1 of v_mfma_f32_32x32x16_bf16 in
+// roll_kernel, which runs the 64- and 96-row tiles of eight 32-column waves (tile_rolls)
+// and rolls its K loop over the group boundary; what follows holds for both.  Each wave
+// dequantizes its own columns on the matrix cores straight from its 16-byte loads into MFMA
+// B fragments -- bf16_rne((q - z) s), the reference's weights, see dequant_step -- with no
+// LDS round trip, so a weight is dequantized NWM times per workgroup and used for 16 WM
+// rows each time: the dequant work per main MFMA falls as 1 / WM whatever TW is.  The
+// activation tile (BM rows x one 128-deep group) is shared by all waves through LDS: it is
+// brought in by direct-to-LDS 16-byte buffer loads, one to four groups per batch
+// (roll_kernel: one group at a time) with the next batch in flight while one is computed,
+// in a row-major layout whose sixteen 16-byte chunks per row are XOR-swizzled by (row &
+// 15): the 16 lanes reading one fragment chunk (16 consecutive rows) then hit 16 different
+// chunk positions, i.e. all 64 LDS banks once.  The scales and zero words of the
 // workgroup's columns for those groups are staged beside them (two direct-to-LDS loads per
 // group for the whole workgroup, issue_sz_stage), and the weights travel in a matching ring
 // of registers.

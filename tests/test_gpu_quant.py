@@ -51,8 +51,8 @@ def test_ties_round_half_to_even(cal):
 @pytest.mark.parametrize("out_f,in_f,gs", [(136, 256, 128), (64, 64, 2), (8, 384, 128), (1000, 512, 64),
                                            (200, 96, 32)])
 def test_bit_exact_against_oracle(cal, dtype, out_f, in_f, gs):
-    """Partial 64-row workgroups (136, 200, 1000 rows), small and large groups, every
-    weight dtype; weights with outlier rows and a constant row (max - min = 0 -> 1e-5)."""
+    """Partial workgroups of 128 rows (groups of 32, 64 and 128) and of 64 (other groups), small
+    and large groups, every weight dtype; weights with outlier rows and a constant row (max - min = 0 -> 1e-5)."""
     gen = torch.Generator().manual_seed(out_f + in_f + gs)
     w = torch.randn((out_f, in_f), generator=gen) * 0.05
     w[3] *= 40.0
